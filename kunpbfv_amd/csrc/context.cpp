@@ -299,38 +299,77 @@ std::vector<kbfv_tw> tws(const std::vector<uint64_t> &v, const std::vector<uint6
     return r;
 }
 
-// int8-MFMA operand tables.  For a K x J matrix M mod p_j: the expanded matrix
-// [JP][8][KP] of packed digit bytes (entry E[j][v][i] packs, in byte u, digit
-// v of the balanced digits of 2^(8u) M_ij mod p_j), padded to 16 ceil(J/16)
-// rows and 8 ceil(K/8) columns with zeros; then per output row j KB_MX_ROW
-// words: the offset (-KB_MX_ACC_BIAS * sum_v 2^(8v)) mod p_j that cancels the
-// accumulator bias, 2^64 - p_j, the offset and 1/p_j as doubles, and the
+// Operand table of the register conversion kernels: K x J entries mod p_j and
+// one extra row (the overflow count's [-Q]_p of a base conversion, which is not
+// offset by 2^59; the diagonal of scale-and-round, which is).
+template <class Entry, class Extra>
+std::vector<uint64_t> conv_table(int K, int J, const std::vector<uint64_t> &pj, bool extra_offset, Entry entry,
+                                 Extra extra) {
+    const int RW = kb_conv_row_words(K);
+    std::vector<uint64_t> v((size_t)RW * J, 0);
+    for (int j = 0; j < J; j++) {
+        uint64_t *row = v.data() + (size_t)RW * j;
+        const uint64_t p = pj[j];
+        uint64_t sum = 0;  // of the rows whose operand is offset, mod p
+        for (int i = 0; i <= K; i++) {
+            const uint64_t m = (i < K ? entry(i, j) : extra(j)) % p;
+            if (i < K || extra_offset) sum = (sum + m) % p;
+            const int64_t s = m > p / 2 ? (int64_t)m - (int64_t)p : (int64_t)m;
+            const int64_t m1 = (s + (1LL << 29)) >> 30, m0 = s - m1 * (1LL << 30);
+            const int32_t w[3] = {(int32_t)m0, (int32_t)m1, (int32_t)(m0 + m1)};
+            std::memcpy((uint8_t *)row + 12 * (size_t)i, w, 12);
+        }
+        int s = 0;
+        while (p >> s) s++;
+        const uint64_t w = (uint64_t)(((kb_u128_host)1 << s) % p);
+        const uint64_t bias = mulmod((1ULL << 63) % p, w, p);  // what the sign flip of the quotient adds
+        uint64_t *c = row + (RW - KB_CONV_TAIL);
+        c[0] = (mulmod((1ULL << 59) % p, sum, p) + p - bias) % p;
+        c[1] = w, c[2] = shoup(w, p), c[3] = 0 - p, c[4] = 0 - 2 * p, c[5] = 0 - 4 * p, c[6] = (uint64_t)s;
+    }
+    return v;
+}
+
+std::vector<kb_conv_in> conv_inputs(const std::vector<uint64_t> &v, const std::vector<uint64_t> &mods) {
+    std::vector<kb_conv_in> r(v.size());
+    for (size_t i = 0; i < v.size(); i++) r[i] = {v[i], shoup(v[i], mods[i]), 0 - mods[i], 0 - 2 * mods[i]};
+    return r;
+}
+
+// int8-MFMA operand tables (rns_mfma.hip).  For a K x J matrix M mod p_j the
+// expanded entry E[j][v][i] packs, in byte u, digit v of the balanced digits of
+// 2^(8u) M_ij mod p_j, padded to 16 ceil(J/16) rows and 8 ceil(K/8) columns with
+// zeros and stored as the kernel's lanes read it: [16-row tile][v][8-column
+// chunk][lane] pairs, lane 16 g + r holding row r, columns 2g and 2g + 1.  Then per
+// output row KB_MX_ROW words: the offset (-KB_MX_ACC_BIAS * sum_v 2^(8v)) mod p_j
+// that cancels the accumulator bias, 2^64 - p_j, the quotient factor, and the
 // diagonal coefficient of scale-and-round with its Shoup companion.
 template <class Entry, class Diag>
 std::vector<uint64_t> mfma_table(int K, int J, const std::vector<uint64_t> &pj, Entry entry, Diag diag) {
-    const int KP = 8 * ((K + 7) / 8), JP = 16 * ((J + 15) / 16);
-    std::vector<uint64_t> v((size_t)JP * 8 * KP + KB_MX_ROW * (size_t)JP, 0);
+    const int KC = (K + 7) / 8, NJ = (J + 15) / 16;
+    const size_t words = (size_t)NJ * 8 * KC * 64 * 2;
+    std::vector<uint64_t> v(words + KB_MX_ROW * 16 * (size_t)NJ, 0);
     kb_u128_host bias_sum = 0;
     for (int u = 0; u < 8; u++) bias_sum += (kb_u128_host)KB_MX_ACC_BIAS << (8 * u);
     for (int j = 0; j < J; j++) {
+        const uint64_t p = pj[j];
         for (int i = 0; i < K; i++) {
-            const uint64_t m = entry(i, j) % pj[j];
+            const uint64_t m = entry(i, j) % p;
+            const int c = i / 8, lane = 16 * (i % 8 / 2) + j % 16;
             for (int u = 0; u < 8; u++) {
-                const uint64_t mu = (uint64_t)(((kb_u128_host)m << (8 * u)) % pj[j]);
+                const uint64_t mu = (uint64_t)(((kb_u128_host)m << (8 * u)) % p);
                 const uint64_t d = (mu + KB_DIGIT_BIAS) ^ KB_DIGIT_BIAS;
-                for (int w = 0; w < 8; w++) v[((size_t)j * 8 + w) * KP + i] |= ((d >> (8 * w)) & 0xff) << (8 * u);
+                for (int w = 0; w < 8; w++)
+                    v[((((size_t)(j / 16) * 8 + w) * KC + c) * 64 + lane) * 2 + i % 2] |= ((d >> (8 * w)) & 0xff)
+                                                                                           << (8 * u);
             }
         }
-        uint64_t *row = v.data() + (size_t)JP * 8 * KP + KB_MX_ROW * (size_t)j;
-        const uint64_t off = (pj[j] - (uint64_t)(bias_sum % pj[j])) % pj[j];
-        const double offd = (double)off, invp = 1.0 / (double)pj[j];
-        const uint64_t dg = diag(j) % pj[j];
-        row[0] = off;
-        row[1] = 0 - pj[j];
-        std::memcpy(&row[2], &offd, 8);
-        std::memcpy(&row[3], &invp, 8);
-        row[4] = dg;
-        row[5] = shoup(dg, pj[j]);
+        uint64_t *row = v.data() + words + KB_MX_ROW * (size_t)j;
+        const uint64_t dg = diag(j) % p;
+        row[0] = (p - (uint64_t)(bias_sum % p)) % p;
+        row[1] = 0 - p;
+        row[2] = (uint64_t)(((kb_u128_host)1 << (80 + KB_MX_QSHIFT)) / p);
+        row[3] = dg, row[4] = shoup(dg, p);
     }
     return v;
 }
@@ -339,15 +378,15 @@ std::vector<uint64_t> mfma_table(int K, int J, const std::vector<uint64_t> &pj, 
 // that goes with it): HPS base conversion Q <-> R and scale-and-round
 // (include/BasisConv_QR.cuh:53-189, include/BFVcontext.cuh:1268-1388), HPS
 // decryption (:1024-1137), the encryption constant -Q mod t (:881-924) and the
-// int8-MFMA operands of the first two.  Built once for the full Q and once
+// register kernels' operands of the first two.  Built once for the full Q and once
 // per level view (Q_l, R_l).
 struct LevelTables {
     std::vector<uint64_t> q_hatinv, q_hat_mod_r, alphaQ, r_hatinv, r_hat_mod_q, alphaR, sr_modr;
     std::vector<double> q_inv, r_inv, sr_frac, dec_frac, dec_B_frac;
-    std::vector<uint64_t> dec_modt, dec_B_modt, q_hatinv_n, mx_qr, mx_rq, mx_sr;
+    std::vector<uint64_t> dec_modt, dec_B_modt, q_hatinv_n, cv_qr, cv_rq, cv_sr, mx_qr, mx_rq, mx_sr;
     int qMSB = 0, sizeQMSB = 0, tMSB = 0;
     uint64_t negQ_mod_t = 0;
-    bool mx_ok = false;
+    bool cv_ok = false, mx_ok = false;
 };
 
 LevelTables level_tables(const std::vector<uint64_t> &Q, const std::vector<uint64_t> &R, uint64_t plain, int N) {
@@ -417,30 +456,42 @@ LevelTables level_tables(const std::vector<uint64_t> &Q, const std::vector<uint6
     // [q_hatinv n^-1]_q for inputs that are N times the INTT
     L.q_hatinv_n.resize(qn);
     for (int i = 0; i < qn; i++) L.q_hatinv_n[i] = mulmod(L.q_hatinv[i], invmod((uint64_t)N % Q[i], Q[i]), Q[i]);
-    // every matrix of the MFMA path has K, J <= 32, and its epilogue's quotient
-    // estimate needs output primes of at least 2^58
-    L.mx_ok = rn + 1 <= 32;
+    // the register kernels hold rn = qn + 1 inputs at most
+    L.cv_ok = rn <= KB_CONV_MAXROWS;
+    if (L.cv_ok) {
+        L.cv_qr = conv_table(
+            qn, rn, R, false, [&](int i, int j) { return L.q_hat_mod_r[j * qn + i]; },
+            [&](int j) { return R[j] - L.alphaQ[rn + j]; });
+        L.cv_rq = conv_table(
+            rn, qn, Q, false, [&](int i, int j) { return L.r_hat_mod_q[j * rn + i]; },
+            [&](int j) { return Q[j] - L.alphaR[qn + j]; });
+        L.cv_sr = conv_table(
+            qn, rn, R, true, [&](int i, int j) { return L.sr_modr[j * (qn + 1) + i]; },
+            [&](int j) { return L.sr_modr[j * (qn + 1) + qn]; });
+    }
+    // the matrix kernel: K, J <= 32 and a quotient below 2^22, so output primes of
+    // at least 2^58
+    L.mx_ok = qn >= KB_MX_MIN_Q && rn + 1 <= 32;
     for (uint64_t m : Q) L.mx_ok = L.mx_ok && m >= (1ULL << 58);
     for (uint64_t m : R) L.mx_ok = L.mx_ok && m >= (1ULL << 58);
     if (L.mx_ok) {
         auto none = [](int) { return (uint64_t)0; };
         L.mx_qr = mfma_table(
             qn + 1, rn, R,
-            [&](int i, int j) { return i < qn ? L.q_hat_mod_r[j * qn + i] : (R[j] - L.alphaQ[rn + j]) % R[j]; },
-            none);
+            [&](int i, int j) { return i < qn ? L.q_hat_mod_r[j * qn + i] : R[j] - L.alphaQ[rn + j]; }, none);
         L.mx_rq = mfma_table(
             rn + 1, qn, Q,
-            [&](int i, int j) { return i < rn ? L.r_hat_mod_q[j * rn + i] : (Q[j] - L.alphaR[qn + j]) % Q[j]; },
-            none);
+            [&](int i, int j) { return i < rn ? L.r_hat_mod_q[j * rn + i] : Q[j] - L.alphaR[qn + j]; }, none);
         L.mx_sr = mfma_table(
-            qn, rn, R, [&](int i, int j) { return L.sr_modr[j * (qn + 1) + i]; },
+            qn + 2, rn, R,
+            [&](int i, int j) { return i < qn ? L.sr_modr[j * (qn + 1) + i] : i == qn ? 1 : 1ULL << 32; },
             [&](int j) { return L.sr_modr[j * (qn + 1) + qn]; });
     }
     return L;
 }
 
 struct LevelOffsets {
-    size_t qhi, qhr, aq, qinv, rhi, rhq, ar, rinv, srm, srf, dm, df, dbm, dbf, qhin, mxqr, mxrq, mxsr;
+    size_t qhi, qhr, aq, qinv, rhi, rhq, ar, rinv, srm, srf, dm, df, dbm, dbf, qhin, ciq, ciqn, cir, cvqr, cvrq, cvsr, mxqr, mxrq, mxsr;
 };
 
 LevelOffsets add_level(Blob &b, const LevelTables &L, const std::vector<uint64_t> &Q,
@@ -455,11 +506,14 @@ LevelOffsets add_level(Blob &b, const LevelTables &L, const std::vector<uint64_t
     o.dm = b.add(tws(L.dec_modt, tvec_plain)), o.df = b.add(L.dec_frac);
     o.dbm = b.add(tws(L.dec_B_modt, tvec_plain)), o.dbf = b.add(L.dec_B_frac);
     o.qhin = b.add(tws(L.q_hatinv_n, Q));
+    o.ciq = b.add(conv_inputs(L.q_hatinv, Q)), o.ciqn = b.add(conv_inputs(L.q_hatinv_n, Q));
+    o.cir = b.add(conv_inputs(L.r_hatinv, R));
+    o.cvqr = b.add(L.cv_qr), o.cvrq = b.add(L.cv_rq), o.cvsr = b.add(L.cv_sr);
     o.mxqr = b.add(L.mx_qr), o.mxrq = b.add(L.mx_rq), o.mxsr = b.add(L.mx_sr);
     return o;
 }
 
-void bind_level(kb_dev_tables &d, const uint8_t *base, const LevelOffsets &o, bool mx_ok) {
+void bind_level(kb_dev_tables &d, const uint8_t *base, const LevelOffsets &o, bool cv_ok, bool mx_ok) {
     auto at = [&](size_t off) { return (const void *)(base + off); };
     d.q_hatinv = (const kbfv_tw *)at(o.qhi), d.q_hat_mod_r = (const uint64_t *)at(o.qhr);
     d.alphaQ_mod_r = (const uint64_t *)at(o.aq), d.q_inv = (const double *)at(o.qinv);
@@ -469,6 +523,11 @@ void bind_level(kb_dev_tables &d, const uint8_t *base, const LevelOffsets &o, bo
     d.dec_modt = (const kbfv_tw *)at(o.dm), d.dec_frac = (const double *)at(o.df);
     d.dec_B_modt = (const kbfv_tw *)at(o.dbm), d.dec_B_frac = (const double *)at(o.dbf);
     d.q_hatinv_n = (const kbfv_tw *)at(o.qhin);
+    d.cv_in_q = (const kb_conv_in *)at(o.ciq), d.cv_in_qn = (const kb_conv_in *)at(o.ciqn);
+    d.cv_in_r = (const kb_conv_in *)at(o.cir);
+    d.cv_qr = cv_ok ? (const uint64_t *)at(o.cvqr) : nullptr;
+    d.cv_rq = cv_ok ? (const uint64_t *)at(o.cvrq) : nullptr;
+    d.cv_sr = cv_ok ? (const uint64_t *)at(o.cvsr) : nullptr;
     d.mx_qr = mx_ok ? (const uint64_t *)at(o.mxqr) : nullptr;
     d.mx_rq = mx_ok ? (const uint64_t *)at(o.mxrq) : nullptr;
     d.mx_sr = mx_ok ? (const uint64_t *)at(o.mxsr) : nullptr;
@@ -738,7 +797,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
     kb_dev_tables &d = c->t;
     d.mod = (const uint64_t *)at(o_mod), d.mu = (const uint64_t *)at(o_mu);
     d.tw = c->d_tw, d.ninv = (const kbfv_tw *)at(o_ninv);
-    bind_level(d, (const uint8_t *)c->d_blob, o_lvl, L0.mx_ok);
+    bind_level(d, (const uint8_t *)c->d_blob, o_lvl, L0.cv_ok, L0.mx_ok);
     d.tinv_mod_q = (const kbfv_tw *)at(o_ti);
     d.ri_hatinv = (const kbfv_tw *)at(o_rih), d.ri_hat_mod_t = (const uint64_t *)at(o_rht);
     d.ri_mod_t = (const uint64_t *)at(o_rmt);
@@ -804,7 +863,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
             free_context(c);
             return KBFV_EHIP;
         }
-        bind_level(v->t, (const uint8_t *)v->d_level_blob, ol, Ll.mx_ok);
+        bind_level(v->t, (const uint8_t *)v->d_level_blob, ol, Ll.cv_ok, Ll.mx_ok);
         const uint8_t *vb = (const uint8_t *)v->d_level_blob;
         v->t.qj_hatinv = (const kbfv_tw *)(vb + o_lqh);
         v->t.qj_hat_mod_t = (const uint64_t *)(vb + o_lqht);

@@ -130,3 +130,52 @@ __device__ __forceinline__ uint64_t kb_csub_s(uint64_t a, uint64_t b) {
     const uint64_t t = a - b;
     return (int64_t)t < 0 ? a : t;
 }
+
+// 64-bit value + 32-bit value as one v_mad_u64_u32 (b * 1 + a): no carry
+// through an SGPR and no register pair to build for b
+__device__ __forceinline__ uint64_t kb_add_u32(uint64_t a, uint32_t b) {
+    uint32_t one = 1;
+    asm("" : "+s"(one));  // a multiplier the optimizer cannot fold away
+    return kb_mad32(b, one, a);
+}
+
+// Shoup product x*w mod q with an under-estimated quotient, in [0, 4q) for any
+// x < 2^64.  floor(x*ws / 2^64) = x1*s1 + hi(x1*s0) + hi(x0*s1) + e with
+// e in {0, 1, 2} (the carries of the low words and hi(x0*s0)); leaving e out
+// adds at most 2q to the lazy residue x*w - h*q in [0, 2q).  nq = 2^64 - q.
+__device__ __forceinline__ uint64_t kb_shoup4(uint64_t x, uint64_t w, uint64_t ws, uint64_t nq) {
+    const uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32);
+    const uint32_t s0 = (uint32_t)ws, s1 = (uint32_t)(ws >> 32);
+    const uint64_t h = kb_add_u32(kb_mad32(x1, s1, __umulhi(x1, s0)), __umulhi(x0, s1));
+    const uint32_t h0 = (uint32_t)h, h1 = (uint32_t)(h >> 32);
+    const uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
+    const uint32_t n0 = (uint32_t)nq, n1 = (uint32_t)(nq >> 32);
+    const uint64_t r = kb_mad32(h0, n0, kb_mad32(x0, w0, 0));
+    const uint32_t cross = kb_mul_lo32(x0, w1) + kb_mul_lo32(x1, w0) + kb_mul_lo32(h0, n1) +
+                           kb_mul_lo32(h1, n0);
+    return r + ((uint64_t)cross << 32);
+}
+
+// a >= m ? a - m : a for a, m < 2^63, given nm = 2^64 - m: the sign of a - m
+// selects word by word (v_bfi_b32), no compare or carry through an SGPR
+__device__ __forceinline__ uint64_t kb_csub_sel(uint64_t a, uint64_t nm) {
+    const uint64_t t = a + nm;
+    const uint32_t msk = (uint32_t)((int32_t)(uint32_t)(t >> 32) >> 31);
+    uint32_t lo, hi;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(lo) : "v"(msk), "v"((uint32_t)a), "v"((uint32_t)t));
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(hi) : "v"(msk), "v"((uint32_t)(a >> 32)), "v"((uint32_t)(t >> 32)));
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Signed 30-bit halves of a residue x < 2^60: x - 2^59 = x1 2^30 + x0 with
+// x0 in [-2^29, 2^29), x1 in [-2^29, 2^29].
+__device__ __forceinline__ void kb_split30(uint64_t x, int &x0, int &x1) {
+    const uint64_t z = x + (1ULL << 29);
+    x0 = (int)((uint32_t)z & 0x3fffffffu) - (1 << 29);
+    x1 = (int)(uint32_t)(z >> 30) - (1 << 29);
+}
+// acc += a*m (wrap-around) with a wave-uniform m.  Opaque to the compiler, which
+// keeps the operands of the plain expression sign-extended in register pairs.
+__device__ __forceinline__ void kb_mad_sv(int64_t &acc, int a, int m) {
+    asm("v_mad_i64_i32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(a), "s"(m) : "vcc");
+}

@@ -43,6 +43,12 @@ void kb_set_error(const char *fmt, ...);
         }                                                                                    \
     } while (0)
 
+// one input limb of a base conversion: (Q/q)^-1 mod q with its Shoup companion,
+// 2^64 - q and 2^64 - 2q
+struct kb_conv_in {
+    uint64_t w, ws, nq, n2q;
+};
+
 // ---------------------------------------------------------------- context
 // Device pointers of every precomputed table.  Small tables live in one
 // device allocation (blob); twiddles in their own.
@@ -89,11 +95,15 @@ struct kb_dev_tables {
     const uint64_t *P_mod_q;         // [qn]
     // modulus switching: [l][i] = q_l^-1 mod q_i (with Shoup companion), i < l
     const kbfv_tw *ql_inv_mod_qi;    // [qn][qn]
-    // int8-MFMA operand tables: [16*ceil(J/16)][8][8*ceil(K/8)] packed digits of
-    // 2^(8u) M_ij mod p_j, then [16*ceil(J/16)][2] offsets (null if too large)
-    const uint64_t *mx_qr;  // base conversion Q -> R, K = qn + 1 (alpha row [-Q]_r)
-    const uint64_t *mx_rq;  // base conversion R -> Q, K = rn + 1 (alpha row [-R]_q)
-    const uint64_t *mx_sr;  // scale-and-round, K = qn
+    // a conversion's input constants: [x (Q/q_i)^-1]_{q_i}, with n^-1 folded in (qn), and R's
+    const kb_conv_in *cv_in_q, *cv_in_qn, *cv_in_r;
+    // operand tables of the register kernels (rns_conv.hip), rows of
+    // kb_conv_row_words(inputs) words (null if the chain is too long for them)
+    const uint64_t *cv_qr;  // base conversion Q -> R
+    const uint64_t *cv_rq;  // base conversion R -> Q
+    const uint64_t *cv_sr;  // scale-and-round
+    // operand tables of the matrix kernel (rns_mfma.hip; null if the chain is not for it)
+    const uint64_t *mx_qr, *mx_rq, *mx_sr;
     // SEAL slot order: NTT index of slot i (batching only, else null)
     const uint64_t *seal_map;  // [N]
     // for inputs that are N times the INTT (kb_intt_noscale): n^-1 folded in
@@ -102,6 +112,13 @@ struct kb_dev_tables {
     const uint64_t *halfT_n;    // [tn] [N (T/2 mod t)]_t
     const kbfv_tw *inv_w1;      // [nmod] inverse table entry 1 without its n^-1
 };
+
+// Rows of a conversion table (rns_conv.hip), in 64-bit words: the signed 30-bit
+// halves of every matrix entry and of one extra row with their sums (three int
+// each), then the constant, 2^s mod p with its Shoup companion, 2^64 - p,
+// 2^64 - 2p, 2^64 - 4p and s.
+constexpr int KB_CONV_MAXROWS = 31, KB_CONV_TAIL = 7;
+__host__ __device__ constexpr int kb_conv_row_words(int in_n) { return (3 * in_n + 4) / 2 + KB_CONV_TAIL; }
 
 struct kbfv_context {
     int log_n = 0, n = 0;

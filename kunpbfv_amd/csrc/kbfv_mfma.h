@@ -46,8 +46,15 @@ typedef int kb_v4i __attribute__((ext_vector_type(4)));
 // biased sums lie in [0, 2^23] and pairs of them combine as unsigned 32-bit
 // words.  The table's per-row offset cancels the bias modulo p.
 #define KB_MX_ACC_BIAS (1 << 22)
-// words per output row after the expanded matrix
-#define KB_MX_ROW 6
+// words per output row after the expanded matrix; binary places of its quotient
+// factor below the top 32 bits of the 80-bit sum
+#define KB_MX_ROW 5
+#define KB_MX_QSHIFT 9
+// shortest chain the matrix kernel takes.  Q -> R and R -> Q of 64 polynomials
+// at N = 2^15, matrix against register kernel: 106 + 112 against 100 + 108 us with
+// 10 primes, 107 + 123 against 113 + 131 us with 11, 115 + 131 against 143 + 172 us
+// with 13 (scale-and-round turns at 12).
+#define KB_MX_MIN_Q 11
 
 __device__ __forceinline__ uint64_t kb_digits(uint64_t x) { return (x + KB_DIGIT_BIAS) ^ KB_DIGIT_BIAS; }
 

@@ -18,11 +18,15 @@ int kb_hps_decrypt(const kbfv_context *c, const uint64_t *x, uint64_t *m, int ba
 int kb_delta_m(const kbfv_context *c, const uint64_t *m, uint64_t *out, int batch, hipStream_t st);
 int kb_reduce_plain(const kbfv_context *c, uint64_t *v, long count, hipStream_t st);
 
-// rns_mfma.hip: the same base conversion and scale-and-round on the int8 matrix
-// cores; return 1 (nothing launched) when the bases are too large for them
-bool kb_rns_gemm_fits(int k_rows, int out_n);
+// rns_conv.hip: the same base conversion and scale-and-round with a
+// coefficient's input limbs in registers (at most KB_CONV_MAXROWS rows)
+int kb_bconv_reg(const kbfv_context *c, bool q_to_r, const uint64_t *x, long in_stride, uint64_t *y,
+                 long out_stride, int polys, hipStream_t st, bool noscale);
+int kb_scale_round_reg(const kbfv_context *c, const uint64_t *x, uint64_t *y, int polys, hipStream_t st);
+
+// rns_mfma.hip: the same on the int8 matrix cores
 int kb_bconv_mfma(const kbfv_context *c, bool q_to_r, const uint64_t *x, long in_stride, uint64_t *y,
-                  long out_stride, int polys, hipStream_t st, bool noscale = false);
+                  long out_stride, int polys, hipStream_t st, bool noscale);
 int kb_scale_round_mfma(const kbfv_context *c, const uint64_t *x, uint64_t *y, int polys, hipStream_t st);
 
 // ks.hip

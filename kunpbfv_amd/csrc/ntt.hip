@@ -64,56 +64,20 @@ struct Geo {
     }
 };
 
-// 64-bit value + 32-bit value as one v_mad_u64_u32 (b * 1 + a): no carry
-// through an SGPR and no register pair to build for b
-__device__ __forceinline__ uint64_t add_u32(uint64_t a, uint32_t b) {
-    uint32_t one = 1;
-    asm("" : "+s"(one));  // a multiplier the optimizer cannot fold away
-    return kb_mad32(b, one, a);
-}
-
-// Shoup product x*w mod q with an under-estimated quotient, in [0, 4q) for any
-// x < 2^64.  floor(x*ws / 2^64) = x1*s1 + hi(x1*s0) + hi(x0*s1) + e with
-// e in {0, 1, 2} (the carries of the low words and hi(x0*s0)); leaving e out
-// adds at most 2q to the lazy residue x*w - h*q in [0, 2q).  nq = 2^64 - q.
-__device__ __forceinline__ uint64_t shoup4(uint64_t x, uint64_t w, uint64_t ws, uint64_t nq) {
-    const uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32);
-    const uint32_t s0 = (uint32_t)ws, s1 = (uint32_t)(ws >> 32);
-    const uint64_t h = add_u32(kb_mad32(x1, s1, __umulhi(x1, s0)), __umulhi(x0, s1));
-    const uint32_t h0 = (uint32_t)h, h1 = (uint32_t)(h >> 32);
-    const uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
-    const uint32_t n0 = (uint32_t)nq, n1 = (uint32_t)(nq >> 32);
-    const uint64_t r = kb_mad32(h0, n0, kb_mad32(x0, w0, 0));
-    const uint32_t cross = kb_mul_lo32(x0, w1) + kb_mul_lo32(x1, w0) + kb_mul_lo32(h0, n1) +
-                           kb_mul_lo32(h1, n0);
-    return r + ((uint64_t)cross << 32);
-}
-
-// a >= m ? a - m : a for a, m < 2^63, given nm = 2^64 - m: the sign of a - m
-// selects word by word (v_bfi_b32), no compare or carry through an SGPR
-__device__ __forceinline__ uint64_t csub_sel(uint64_t a, uint64_t nm) {
-    const uint64_t t = a + nm;
-    const uint32_t msk = (uint32_t)((int32_t)(uint32_t)(t >> 32) >> 31);
-    uint32_t lo, hi;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(lo) : "v"(msk), "v"((uint32_t)a), "v"((uint32_t)t));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(hi) : "v"(msk), "v"((uint32_t)(a >> 32)), "v"((uint32_t)(t >> 32)));
-    return ((uint64_t)hi << 32) | lo;
-}
-
 // forward values stay in [0, 8q), inverse values in [0, 4q); q < 2^60 keeps
 // every sum below 2^63.  nq = 2^64 - q, q4 = 4q, nq4 = 2^64 - 4q.
 __device__ __forceinline__ void ct_bfly(uint64_t &a, uint64_t &b, kbfv_tw w, uint64_t nq, uint64_t q4,
                                         uint64_t nq4) {
-    a = csub_sel(a, nq4);                        // [0, 4q)
-    const uint64_t t = shoup4(b, w.w, w.ws, nq);  // [0, 4q)
+    a = kb_csub_sel(a, nq4);                        // [0, 4q)
+    const uint64_t t = kb_shoup4(b, w.w, w.ws, nq);  // [0, 4q)
     b = a + q4 - t;                              // (0, 8q)
     a = a + t;                                   // [0, 8q)
 }
 
 __device__ __forceinline__ void gs_bfly(uint64_t &a, uint64_t &b, kbfv_tw w, uint64_t nq, uint64_t q4,
                                         uint64_t nq4) {
-    const uint64_t u = csub_sel(a + b, nq4);               // [0, 4q)
-    const uint64_t v = shoup4(a + q4 - b, w.w, w.ws, nq);  // [0, 4q)
+    const uint64_t u = kb_csub_sel(a + b, nq4);               // [0, 4q)
+    const uint64_t v = kb_shoup4(a + q4 - b, w.w, w.ws, nq);  // [0, 4q)
     a = u;
     b = v;
 }
@@ -237,7 +201,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
 #pragma unroll
                     for (int i = i0; i < i0 + h; ++i) {
                         gs_bfly(x[i], x[i + h], w, nq, q4, nq4);
-                        if (NINV && gst == 0) x[i] = shoup4(x[i], ninv.w, ninv.ws, nq);
+                        if (NINV && gst == 0) x[i] = kb_shoup4(x[i], ninv.w, ninv.ws, nq);
                     }
                 }
             }
@@ -247,9 +211,9 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
             if constexpr (GOUT) {
                 uint64_t v = x[i];
                 if constexpr (FIN) {
-                    if constexpr (FWD) v = csub_sel(v, nq4);
-                    v = csub_sel(v, 0 - (q << 1));
-                    v = csub_sel(v, nq);
+                    if constexpr (FWD) v = kb_csub_sel(v, nq4);
+                    v = kb_csub_sel(v, 0 - (q << 1));
+                    v = kb_csub_sel(v, nq);
                 }
                 gout[posc + (kbase + i * d) * pstep] = v;
             } else {
@@ -358,9 +322,9 @@ __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__rest
         const int c = e / S, k = e % S;
         uint64_t v = tile[G::addr(c, k)];
         if constexpr (LAST) {
-            v = csub_sel(v, 0 - (q << 2));
-            v = csub_sel(v, 0 - (q << 1));
-            v = csub_sel(v, 0 - q);
+            v = kb_csub_sel(v, 0 - (q << 2));
+            v = kb_csub_sel(v, 0 - (q << 1));
+            v = kb_csub_sel(v, 0 - q);
         }
         out[(grp0 * C + c) * S + k] = v;
     }
@@ -540,9 +504,9 @@ __global__ void __launch_bounds__((1 << LOG_N) >> LOG_R)
         for (int j = 0; j < n / T; ++j) {
             const int k = threadIdx.x + j * T;
             uint64_t v = tile[G::addr(0, k)];
-            v = csub_sel(v, 0 - (q << 2));
-            v = csub_sel(v, 0 - (q << 1));
-            v = csub_sel(v, 0 - q);
+            v = kb_csub_sel(v, 0 - (q << 2));
+            v = kb_csub_sel(v, 0 - (q << 1));
+            v = kb_csub_sel(v, 0 - q);
             out[k] = v;
         }
     } else {

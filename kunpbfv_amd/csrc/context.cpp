@@ -336,6 +336,19 @@ std::vector<kb_conv_in> conv_inputs(const std::vector<uint64_t> &v, const std::v
     return r;
 }
 
+std::vector<kb_fold> folds(const std::vector<uint64_t> &mods) {
+    std::vector<kb_fold> r(mods.size());
+    for (size_t i = 0; i < mods.size(); i++) {
+        const uint64_t p = mods[i];
+        int s = 0;
+        while (p >> s) s++;
+        const uint64_t w = (uint64_t)(((kb_u128_host)1 << s) % p);
+        const uint64_t wtop = mulmod(w, (uint64_t)(((kb_u128_host)1 << 64) % p), p);
+        r[i] = {w, shoup(w, p), 0 - p, 0 - 2 * p, 0 - 4 * p, wtop, (uint64_t)s};
+    }
+    return r;
+}
+
 // int8-MFMA operand tables (rns_mfma.hip).  For a K x J matrix M mod p_j the
 // expanded entry E[j][v][i] packs, in byte u, digit v of the balanced digits of
 // 2^(8u) M_ij mod p_j, padded to 16 ceil(J/16) rows and 8 ceil(K/8) columns with
@@ -772,7 +785,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
     size_t o_qli = blob.add(ql_inv);
     size_t o_seal = blob.add(seal_map);
     size_t o_thn = blob.add(tws(t_hatinv_n, T)), o_hfn = blob.add(halfT_n);
-    size_t o_iw1 = blob.add(inv_w1);
+    size_t o_iw1 = blob.add(inv_w1), o_tf = blob.add(folds(T));
 
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) {
@@ -803,6 +816,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
     d.ri_mod_t = (const uint64_t *)at(o_rmt);
     d.qj_hatinv = (const kbfv_tw *)at(o_qjh), d.qj_hat_mod_t = (const uint64_t *)at(o_qjt);
     d.qj_mod_t = (const uint64_t *)at(o_qjm);
+    d.t_fold = (const kb_fold *)at(o_tf);
     d.t_hatinv = (const kbfv_tw *)at(o_th), d.t_hat_mod_pq = (const uint64_t *)at(o_thp);
     d.t_mod_pq = (const uint64_t *)at(o_tmp), d.halfT_mod = (const uint64_t *)at(o_half);
     d.halfT_t = d.halfT_mod + pq;

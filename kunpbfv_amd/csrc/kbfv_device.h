@@ -179,3 +179,32 @@ __device__ __forceinline__ void kb_split30(uint64_t x, int &x0, int &x1) {
 __device__ __forceinline__ void kb_mad_sv(int64_t &acc, int a, int m) {
     asm("v_mad_i64_i32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(a), "s"(m) : "vcc");
 }
+
+// acc += a*b (wrap-around), opaque for the same reason
+__device__ __forceinline__ void kb_mad_vv(uint64_t &acc, uint32_t a, uint32_t b) {
+    asm("v_mad_u64_u32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b) : "vcc");
+}
+// constants of a reduction by folding at bit s, 2^(s-1) < p < 2^s: 2^s mod p with
+// its Shoup companion, 2^64 - p, 2^64 - 2p, 2^64 - 4p, 2^(64+s) mod p, s
+struct kb_fold {
+    uint64_t w, ws, nq, n2q, n4q, wtop, s;
+};
+// (top 2^64 + F) 2^60 + L mod p for L < 2^60 and a value below 64 p^2 (WIDE, top <= 3)
+// or 16 p^2 (top not read)
+template <bool WIDE>
+__device__ __forceinline__ uint64_t kb_fold_reduce(uint64_t F, uint32_t top, uint64_t L, const kb_fold &f) {
+    if (f.s != 60) {  // uniform; then the value is below 2^124: top is 0 here
+        const int s = (int)f.s;
+        top = (uint32_t)(F >> (s + 4));
+        F = (F << (60 - s)) + (L >> s);
+        L &= (1ULL << s) - 1;
+    }
+    uint64_t r = kb_shoup4(F, f.w, f.ws, f.nq) + L;  // [0, 6p)
+    r = kb_csub_sel(r, f.n4q);
+    if constexpr (WIDE) {
+        r = kb_mad32(top, (uint32_t)f.wtop, r) + ((uint64_t)kb_mul_lo32(top, (uint32_t)(f.wtop >> 32)) << 32);
+        r = kb_csub_sel(r, f.n4q);  // [0, 7p) before
+    }
+    r = kb_csub_sel(r, f.n2q);
+    return kb_csub_sel(r, f.nq);
+}

@@ -85,6 +85,7 @@ struct kb_dev_tables {
     const uint64_t *qj_hat_mod_t;    // [dnum][tn][pn]
     const uint64_t *qj_mod_t;        // [dnum][tn]
     const kbfv_tw *t_hatinv;         // [tn]
+    const kb_fold *t_fold;           // [tn]
     const uint64_t *t_hat_mod_pq;    // [pn+qn][tn]
     const uint64_t *t_mod_pq;        // [pn+qn]
     const uint64_t *halfT_mod;       // [pn+qn+tn] in the order P, Q, T

@@ -10,10 +10,7 @@
 //
 // MI355X design: with one special prime (K = 1) the digit decomposition of a
 // limb is the limb itself, so "modUp Qj -> T then NTT over T" is one NTT that
-// reads the Q limb directly (kb_digits_to_t_ntt).  The inner product is
-// key-stationary: each thread holds its key column (2 x dnum values) in
-// registers and walks the whole batch, so the relinearisation key is read from
-// HBM once per call instead of once per ciphertext.
+// reads the Q limb directly (kb_digits_to_t_ntt).
 #include "kbfv_internal.h"
 #include "kbfv_ops.h"
 
@@ -87,107 +84,6 @@ __global__ void k_modup_pq_to_t(kb_dev_tables t, const uint64_t *__restrict__ x,
         kb_sub128(acc, (uint64_t)vf * t.ri_mod_t[kk * B + b]);
         op[(long)kk * n] = kb_barrett128(acc, t.mod[m], t.mu[2 * m], t.mu[2 * m + 1]);
     }
-}
-
-// Key-stationary inner product.  cin [batch][D][tn][N], key [2][KD][KB][tn][N]
-// (read on its first D digits and B blocks: a ciphertext below the full level
-// uses a prefix of the full-level key), out [batch][2][B][tn][N].  A workgroup owns one T limb, 64 coefficients and
-// up to IP_WAVES key blocks (one wave per block b, both key halves in
-// registers).  It walks the whole batch: per ciphertext the D x 64 digit tile
-// is staged once in LDS and read by every wave, so the key is read from HBM
-// once per call and each digit tile ceil(B / IP_WAVES) times.
-constexpr int IP_WAVES = 8;
-template <int MAXD>
-__global__ void __launch_bounds__(64 * IP_WAVES)
-    k_inner_product(kb_dev_tables t, const uint64_t *__restrict__ cin, const uint64_t *__restrict__ key,
-                    uint64_t *__restrict__ out, int D, int B, int KD, int KB, int tn, int oT, int n,
-                    int batch) {
-    __shared__ uint64_t cs[MAXD][64];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int bgroups = (B + IP_WAVES - 1) / IP_WAVES;
-    const int tiles = n / 64;
-    int bid = blockIdx.x;
-    const int bg = bid % bgroups;
-    bid /= bgroups;
-    const int tile = bid % tiles;
-    const int kk = bid / tiles;
-    const int b = bg * IP_WAVES + wave;
-    const bool active = b < B;
-    const int k = tile * 64 + lane;
-    const int m = oT + kk;
-    const uint64_t q = t.mod[m], mlo = t.mu[2 * m], mhi = t.mu[2 * m + 1];
-    const long N = n;
-    const long kstride = (long)KB * tn * N;  // digit stride in the key
-    uint64_t ka[MAXD], kbv[MAXD];
-#pragma unroll
-    for (int i = 0; i < MAXD; ++i) {
-        ka[i] = 0;
-        kbv[i] = 0;
-        if (active && i < D) {
-            const long off = (long)i * kstride + ((long)b * tn + kk) * N + k;
-            ka[i] = key[off];
-            kbv[i] = key[(long)KD * kstride + off];
-        }
-    }
-    // each thread stages at most ceil(MAXD*64 / (64*IP_WAVES)) digit values per ciphertext
-    constexpr int PER = (MAXD + IP_WAVES - 1) / IP_WAVES;
-    uint64_t pre[PER];
-    auto fetch = [&](int bt) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int i = wave + r * IP_WAVES;
-            if (i < D) pre[r] = cin[(((long)bt * D + i) * tn + kk) * N + tile * 64 + lane];
-        }
-    };
-    fetch(0);
-    for (int bt = 0; bt < batch; ++bt) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int i = wave + r * IP_WAVES;
-            if (i < D) cs[i][lane] = pre[r];
-        }
-        __syncthreads();
-        if (bt + 1 < batch) fetch(bt + 1);
-        if (active) {
-            kbfv_u128 a0{0, 0}, a1{0, 0};
-#pragma unroll
-            for (int i = 0; i < MAXD; ++i) {
-                if (i < D) {
-                    const uint64_t cv = cs[i][lane];
-                    kb_mac128(a0, cv, ka[i]);
-                    kb_mac128(a1, cv, kbv[i]);
-                }
-            }
-            uint64_t *op = out + (long)bt * 2 * B * tn * N + ((long)b * tn + kk) * N + k;
-            op[0] = kb_barrett128(a0, q, mlo, mhi);
-            op[(long)B * tn * N] = kb_barrett128(a1, q, mlo, mhi);
-        }
-        __syncthreads();
-    }
-}
-
-// fallback for dnum > 64: one thread per output, key re-read per ciphertext
-__global__ void k_inner_product_generic(kb_dev_tables t, const uint64_t *__restrict__ cin,
-                                        const uint64_t *__restrict__ key, uint64_t *__restrict__ out,
-                                        int D, int B, int KD, int KB, int tn, int oT, int n, long total) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const long N = n;
-    const int k = (int)(i % n);
-    long rest = i / n;
-    const int kk = (int)(rest % tn);
-    rest /= tn;
-    const int b = (int)(rest % B);
-    rest /= B;
-    const int h = (int)(rest % 2);
-    const long bt = rest / 2;
-    const int m = oT + kk;
-    kbfv_u128 acc{0, 0};
-    for (int d = 0; d < D; ++d)
-        kb_mac128(acc, cin[((bt * D + d) * tn + kk) * N + k],
-                  key[(((long)h * KD + d) * KB + b) * tn * N + (long)kk * N + k]);
-    out[i] = kb_barrett128(acc, t.mod[m], t.mu[2 * m], t.mu[2 * m + 1]);
 }
 
 // in [batch][2][B][tn][N] coefficient form -> out [batch][2][pq][N]
@@ -418,31 +314,15 @@ int kb_modup_pq_to_t(const kbfv_context *c, const uint64_t *x, uint64_t *out, in
 int kb_inner_product(const kbfv_context *c, const uint64_t *cin, const uint64_t *key, uint64_t *out,
                      int batch, hipStream_t st) {
     KB_REQUIRE(c && cin && key && out && batch > 0, "bad inner-product arguments");
-    if (batch >= 16) {  // enough ciphertexts to fill the matrix-core column tiles
+    // the matrix cores pay for long keys and large batches only: 28 digits at N =
+    // 2^16, 40 ciphertexts 4.37 against 4.16 ms, 48 4.45 against 4.94, 128 9.32
+    // against 12.7; 18 digits, 48 ciphertexts 3.25 against 3.71 ms; 13 digits, 64
+    // ciphertexts at N = 2^15 1.22 against 0.73 ms
+    if (c->dnum > 16 && batch >= 44) {
         const int r = kb_inner_product_mfma(c, cin, key, out, batch, st);
         if (r != 1) return r;
     }
-    const int D = c->dnum, B = c->ri_blocks, tn = c->tn, n = c->n;
-    const unsigned grid = (unsigned)((n / 64) * tn * ((B + IP_WAVES - 1) / IP_WAVES));
-#define KB_IP(MD)                                                                                        \
-    hipLaunchKernelGGL(k_inner_product<MD>, dim3(grid), dim3(64 * IP_WAVES), 0, st, c->t, cin, key, out, D, \
-                       B, c->key_dnum, c->key_blocks, tn, c->oT, n, batch)
-    if (D <= 4)
-        KB_IP(4);
-    else if (D <= 8)
-        KB_IP(8);
-    else if (D <= 16)
-        KB_IP(16);
-    else if (D <= 32)
-        KB_IP(32);
-    else {
-        const long total = (long)batch * 2 * B * tn * n;
-        hipLaunchKernelGGL(k_inner_product_generic, dim3(blocks_for(total, KS_BS)), dim3(KS_BS), 0, st, c->t,
-                           cin, key, out, D, B, c->key_dnum, c->key_blocks, tn, c->oT, n, total);
-    }
-#undef KB_IP
-    KB_LAUNCH_CHECK();
-    return KBFV_OK;
+    return kb_inner_product_stream(c, cin, key, out, batch, st);
 }
 
 int kb_modup_t_to_pq(const kbfv_context *c, const uint64_t *in, uint64_t *out, int batch, hipStream_t st) {

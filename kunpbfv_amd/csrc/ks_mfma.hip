@@ -222,12 +222,8 @@ int kb_inner_product_mfma(const kbfv_context *c, const uint64_t *cin, const uint
         KB_LAUNCH_CHECK();                                                                               \
         return KBFV_OK;                                                                                  \
     }
-    KB_IM(1, 1)
-    KB_IM(2, 1)
     KB_IM(3, 1)
     KB_IM(4, 1)
-    KB_IM(1, 2)
-    KB_IM(2, 2)
     KB_IM(3, 2)
     KB_IM(4, 2)
 #undef KB_IM

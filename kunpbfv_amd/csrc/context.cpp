@@ -766,6 +766,42 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
         }
     }
 
+    // external product's auxiliary basis: the largest primes below 2^28 that are 1 mod 2^17
+    std::vector<uint2> aux_tw((size_t)KB_AUX_PRIMES * 2 * N);
+    std::vector<kb_aux_mod> aux_mod(KB_AUX_PRIMES);
+    std::vector<kb_aux_mix> aux_mix(1);
+    std::vector<kb_aux_lift> aux_lift(qn);
+    if (primes_desc(1ULL << 28, 1ULL << 17, KB_AUX_PRIMES, c->aux_p) != KBFV_OK) return fail("no auxiliary basis");
+    {
+        const uint64_t *ap = c->aux_p;
+        auto pair32 = [](uint64_t w, uint64_t p) { return uint2{(uint32_t)w, (uint32_t)((w << 32) / p)}; };
+        for (int k = 0; k < KB_AUX_PRIMES; k++) {
+            const uint64_t p = ap[k], r32 = (1ULL << 32) % p;
+            aux_mod[k] = {(uint32_t)p, (uint32_t)((1ULL << 32) / p), (uint32_t)r32, pair32(r32, p).y};
+            const uint64_t ps = powmod(primitive_root(p), (p - 1) / (2 * (uint64_t)N), p), pi = invmod(ps, p);
+            uint2 *f = aux_tw.data() + (size_t)k * 2 * N, *iv = f + N;
+            uint64_t a = 1, b = 1;
+            for (int i = 0; i < N; i++) {
+                const uint64_t at = bitrev((uint64_t)i, log_n);
+                f[at] = pair32(a, p), iv[at] = pair32(b, p);
+                a = a * ps % p, b = b * pi % p;
+            }
+            for (int j = 0; j < k; j++) {
+                const uint64_t inv = invmod(prod_except({ap, ap + KB_AUX_PRIMES}, j, k, -1, p), p);
+                aux_mix[0].other[k][j] = pair32(inv, p);
+            }
+            const uint64_t own = k ? invmod(prod_except({ap, ap + KB_AUX_PRIMES}, 0, k, -1, p), p) : 1;
+            aux_mix[0].own[k] = pair32(own * invmod((uint64_t)N % p, p) % p, p);
+        }
+        for (int i = 0; i < qn; i++) {
+            const uint64_t q1 = Q[i];
+            auto prod = [&](int n) { return prod_except({ap, ap + KB_AUX_PRIMES}, 0, n, -1, q1); };
+            aux_lift[i] = {(uint64_t)(((kb_u128_host)1 << 64) / q1), prod(2), shoup(prod(2), q1), prod(3),
+                           shoup(prod(3), q1), (q1 - prod(3)) % q1, (q1 - prod(4)) % q1, 0 - q1, 0 - 2 * q1,
+                           0 - 4 * q1};
+        }
+    }
+
     // device upload: one blob for the small tables
     Blob blob;
     size_t o_mod = blob.add(mod), o_mu = blob.add(mu), o_ninv = blob.add(ninv);
@@ -786,6 +822,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
     size_t o_seal = blob.add(seal_map);
     size_t o_thn = blob.add(tws(t_hatinv_n, T)), o_hfn = blob.add(halfT_n);
     size_t o_iw1 = blob.add(inv_w1), o_tf = blob.add(folds(T));
+    size_t o_atw = blob.add(aux_tw), o_amd = blob.add(aux_mod), o_amx = blob.add(aux_mix), o_alf = blob.add(aux_lift);
 
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) {
@@ -817,6 +854,8 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
     d.qj_hatinv = (const kbfv_tw *)at(o_qjh), d.qj_hat_mod_t = (const uint64_t *)at(o_qjt);
     d.qj_mod_t = (const uint64_t *)at(o_qjm);
     d.t_fold = (const kb_fold *)at(o_tf);
+    d.aux_tw = (const uint2 *)at(o_atw), d.aux_mod = (const kb_aux_mod *)at(o_amd);
+    d.aux_mix = (const kb_aux_mix *)at(o_amx), d.aux_lift = (const kb_aux_lift *)at(o_alf);
     d.t_hatinv = (const kbfv_tw *)at(o_th), d.t_hat_mod_pq = (const uint64_t *)at(o_thp);
     d.t_mod_pq = (const uint64_t *)at(o_tmp), d.halfT_mod = (const uint64_t *)at(o_half);
     d.halfT_t = d.halfT_mod + pq;

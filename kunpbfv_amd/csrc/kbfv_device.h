@@ -174,15 +174,18 @@ __device__ __forceinline__ void kb_split30(uint64_t x, int &x0, int &x1) {
     x0 = (int)((uint32_t)z & 0x3fffffffu) - (1 << 29);
     x1 = (int)(uint32_t)(z >> 30) - (1 << 29);
 }
-// acc += a*m (wrap-around) with a wave-uniform m.  Opaque to the compiler, which
-// keeps the operands of the plain expression sign-extended in register pairs.
-__device__ __forceinline__ void kb_mad_sv(int64_t &acc, int a, int m) {
-    asm("v_mad_i64_i32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(a), "s"(m) : "vcc");
+// acc += a*b (wrap-around), one v_mad_i64_i32 / v_mad_u64_u32
+__device__ __forceinline__ void kb_mad(int64_t &acc, int a, int b) {
+    acc = (int64_t)((uint64_t)acc + (uint64_t)((int64_t)a * b));
 }
-
-// acc += a*b (wrap-around), opaque for the same reason
-__device__ __forceinline__ void kb_mad_vv(uint64_t &acc, uint32_t a, uint32_t b) {
-    asm("v_mad_u64_u32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b) : "vcc");
+__device__ __forceinline__ void kb_mad(uint64_t &acc, uint32_t a, uint32_t b) { acc += (uint64_t)a * b; }
+// Marks a 32-bit register value as changed.  A multiplicand that a loop reads in
+// every pass is otherwise widened to 64 bits ahead of the loop and takes a
+// register pair for its whole length.
+template <class T>
+__device__ __forceinline__ void kb_pin(T &x) {
+    static_assert(sizeof(T) == 4, "32-bit registers");
+    asm volatile("" : "+v"(x));
 }
 // constants of a reduction by folding at bit s, 2^(s-1) < p < 2^s: 2^s mod p with
 // its Shoup companion, 2^64 - p, 2^64 - 2p, 2^64 - 4p, 2^(64+s) mod p, s

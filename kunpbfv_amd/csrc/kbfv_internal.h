@@ -43,6 +43,23 @@ void kb_set_error(const char *fmt, ...);
         }                                                                                    \
     } while (0)
 
+// the external product's auxiliary basis (ext_aux.hip): primes below 2^28, each with
+// floor(2^32 / p) and 2^32 mod p with its Shoup companion
+constexpr int KB_AUX_PRIMES = 4;
+struct kb_aux_mod {
+    uint32_t p, one_s, r32, r32_s;
+};
+// mixed radix: digit k is own[k] x_k - sum_{j < k} other[k][j] v_j mod p_k (pairs with
+// Shoup companions), own = n^-1 (p_0 .. p_{k-1})^-1, other = (p_j .. p_{k-1})^-1
+struct kb_aux_mix {
+    uint2 own[KB_AUX_PRIMES], other[KB_AUX_PRIMES][KB_AUX_PRIMES];
+};
+// modulo a ciphertext prime: floor(2^64 / q), p_0 p_1 and p_0 p_1 p_2 with their
+// companions, minus the product of three and of four primes, 2^64 - q, - 2q, - 4q
+struct kb_aux_lift {
+    uint64_t one_s, w2, w2_s, w3, w3_s, neg3, neg4, nq, n2q, n4q;
+};
+
 // one input limb of a base conversion: (Q/q)^-1 mod q with its Shoup companion,
 // 2^64 - q and 2^64 - 2q
 struct kb_conv_in {
@@ -105,6 +122,11 @@ struct kb_dev_tables {
     const uint64_t *cv_sr;  // scale-and-round
     // operand tables of the matrix kernel (rns_mfma.hip; null if the chain is not for it)
     const uint64_t *mx_qr, *mx_rq, *mx_sr;
+    // external product's auxiliary basis
+    const uint2 *aux_tw;           // [KB_AUX_PRIMES][2][N] forward and inverse (unscaled) tables
+    const kb_aux_mod *aux_mod;     // [KB_AUX_PRIMES]
+    const kb_aux_mix *aux_mix;
+    const kb_aux_lift *aux_lift;   // [qn]
     // SEAL slot order: NTT index of slot i (batching only, else null)
     const uint64_t *seal_map;  // [N]
     // for inputs that are N times the INTT (kb_intt_noscale): n^-1 folded in
@@ -150,6 +172,7 @@ struct kbfv_context {
 
     // host copies (exported to parity tests)
     std::vector<uint64_t> mod, psi;
+    uint64_t aux_p[KB_AUX_PRIMES] = {};
     std::vector<std::pair<std::string, std::vector<uint64_t>>> host_u64;
     std::vector<std::pair<std::string, std::vector<double>>> host_f64;
 

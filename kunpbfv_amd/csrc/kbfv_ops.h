@@ -87,3 +87,12 @@ int kb_gadget_mac(const kbfv_context *c, const uint64_t *dig, const uint64_t *rg
                   int batch, int rc, hipStream_t st);
 int kb_rgsw_add_gadget(const kbfv_context *c, uint64_t *rgsw, const uint64_t *m_ntt, int base_bits, int nd,
                        hipStream_t st);
+
+// ext_aux.hip: the external product's sum through the auxiliary basis.  Primes it
+// needs for `rows` rows of base 2^bits (0: it does not fit), rows of one chunk
+// (< 1: the workspace is too small), and the product: coef the coefficient-form
+// ciphertexts, dig_ws 8 qn batch limbs, out also scratch until it is written
+int kb_ext_aux_primes(const kbfv_context *c, int rows, int bits);
+int kb_ext_aux_rows(const kbfv_context *c, int batch, int np);
+int kb_external_product_aux(const kbfv_context *c, const uint64_t *rgsw, const uint64_t *coef, uint64_t *out,
+                            uint64_t *dig_ws, int batch, int rows, int nd, int bits, int np, hipStream_t st);

@@ -117,9 +117,9 @@ __global__ void __launch_bounds__(64 * IS_WAVES)
                         const uint32_t x0 = (uint32_t)x[i][c][v] & M, x1 = (uint32_t)(x[i][c][v] >> 30);
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
-                            kb_mad_vv(lo[c][h][v], x0, k0[h]);
-                            kb_mad_vv(hi[c][h][v], x1, k1[h]);
-                            kb_mad_vv(mm[c][h][v], x0 + x1, k0[h] + k1[h]);
+                            kb_mad(lo[c][h][v], x0, k0[h]);
+                            kb_mad(hi[c][h][v], x1, k1[h]);
+                            kb_mad(mm[c][h][v], x0 + x1, k0[h] + k1[h]);
                         }
                     }
                 }
@@ -231,14 +231,14 @@ __global__ void __launch_bounds__(64 * IS_WAVES)
                 const uint4 x = xs[buf][i][lane];
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    uint32_t ks;  // formed here: kept for the whole batch it would cost a register each
-                    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ks) : "v"(k0[i][h]), "v"(k1[i][h]));
-                    kb_mad_vv(lo[0][h], x.x, k0[i][h]);
-                    kb_mad_vv(lo[1][h], x.z, k0[i][h]);
-                    kb_mad_vv(hi[0][h], x.y, k1[i][h]);
-                    kb_mad_vv(hi[1][h], x.w, k1[i][h]);
-                    kb_mad_vv(mm[0][h], x.x + x.y, ks);
-                    kb_mad_vv(mm[1][h], x.z + x.w, ks);
+                    kb_pin(k0[i][h]), kb_pin(k1[i][h]);  // and their sum is formed here, not kept
+                    const uint32_t ks = k0[i][h] + k1[i][h];
+                    kb_mad(lo[0][h], x.x, k0[i][h]);
+                    kb_mad(lo[1][h], x.z, k0[i][h]);
+                    kb_mad(hi[0][h], x.y, k1[i][h]);
+                    kb_mad(hi[1][h], x.w, k1[i][h]);
+                    kb_mad(mm[0][h], x.x + x.y, ks);
+                    kb_mad(mm[1][h], x.z + x.w, ks);
                 }
             }
             if (i % 8 == 7 || i == MAXD - 1) {

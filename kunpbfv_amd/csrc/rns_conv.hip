@@ -73,6 +73,8 @@ __global__ void __launch_bounds__(256)
     for (int j = 0; j < out_n; ++j) {
         const uint64_t *row = tab + (long)j * RW;
         const int *m = (const int *)row;
+#pragma unroll
+        for (int i = 0; i < IN; ++i) kb_pin(x0[i]), kb_pin(x1[i]), kb_pin(xs[i]);
         uint64_t dnext = 0;
         if (SR) dnext = xp[(IN + min(j + 1, out_n - 1)) * n];
         int64_t lo = 0, hi = 0, mid[NG];
@@ -82,20 +84,20 @@ __global__ void __launch_bounds__(256)
             int64_t mm = 0;
 #pragma unroll
             for (int i = g * G; i < IN && i < g * G + G; ++i) {
-                kb_mad_sv(lo, x0[i], m[3 * i]);
-                kb_mad_sv(hi, x1[i], m[3 * i + 1]);
-                kb_mad_sv(mm, xs[i], m[3 * i + 2]);
+                kb_mad(lo, x0[i], m[3 * i]);
+                kb_mad(hi, x1[i], m[3 * i + 1]);
+                kb_mad(mm, xs[i], m[3 * i + 2]);
             }
             if (g == NG - 1) {  // the last group takes the extra row
                 if constexpr (SR) {
                     int d0, d1;
                     kb_split30(diag, d0, d1);
-                    kb_mad_sv(lo, d0, m[3 * IN]);
-                    kb_mad_sv(hi, d1, m[3 * IN + 1]);
-                    kb_mad_sv(mm, d0 + d1, m[3 * IN + 2]);
+                    kb_mad(lo, d0, m[3 * IN]);
+                    kb_mad(hi, d1, m[3 * IN + 1]);
+                    kb_mad(mm, d0 + d1, m[3 * IN + 2]);
                 } else {
-                    kb_mad_sv(lo, alpha, m[3 * IN]);
-                    kb_mad_sv(mm, alpha, m[3 * IN + 2]);
+                    kb_mad(lo, alpha, m[3 * IN]);
+                    kb_mad(mm, alpha, m[3 * IN + 2]);
                 }
             }
             const uint64_t o = (uint64_t)lo + (uint64_t)hi;

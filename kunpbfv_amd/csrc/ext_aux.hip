@@ -551,11 +551,12 @@ int run(const kbfv_context *c, const uint64_t *rgsw, const uint64_t *coef, uint6
 }  // namespace
 
 // rows of a chunk: its digits fit what the accumulators leave of the digit
-// workspace, its rows in the basis the output less one row's limbs
+// workspace, its rows in the basis the output less an eighth for the limbs on their
+// way there (with room for one row's only, 17 ciphertexts took 1.31 ms, 16 0.82)
 int kb_ext_aux_rows(const kbfv_context *c, int batch, int np) {
     const long hls = 2L * c->qn;
     const long by_dig = (16L * c->qn - hls * np) / np;                 // per ciphertext
-    const long by_key = 2 * (hls * batch - hls) / (hls * np);
+    const long by_key = 2L * (batch - (batch + 7) / 8) / np;
     return (int)std::min(std::min(by_dig, by_key), (long)AM_MAXR);
 }
 

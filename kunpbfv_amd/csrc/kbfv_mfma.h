@@ -50,11 +50,11 @@ typedef int kb_v4i __attribute__((ext_vector_type(4)));
 // factor below the top 32 bits of the 80-bit sum
 #define KB_MX_ROW 5
 #define KB_MX_QSHIFT 9
-// shortest chain the matrix kernel takes.  Q -> R and R -> Q of 64 polynomials
-// at N = 2^15, matrix against register kernel: 106 + 112 against 100 + 108 us with
-// 10 primes, 107 + 123 against 113 + 131 us with 11, 115 + 131 against 143 + 172 us
-// with 13 (scale-and-round turns at 12).
-#define KB_MX_MIN_Q 11
+// shortest chain the matrix kernel takes.  Q -> R, R -> Q and scale-and-round of 64
+// polynomials at N = 2^15, matrix against register kernel: 107, 123, 162 against 98,
+// 109, 139 us with 11 primes; 108, 128, 168 against 114, 131, 153 with 12; 115, 131, 176
+// against 125, 149, 164 with 13 (HomMult takes four of the first to three of each other).
+#define KB_MX_MIN_Q 13
 
 __device__ __forceinline__ uint64_t kb_digits(uint64_t x) { return (x + KB_DIGIT_BIAS) ^ KB_DIGIT_BIAS; }
 

@@ -11,7 +11,7 @@ from test_gpu_rns_sizes import rand_mod
 
 pytestmark = pytest.mark.gpu
 
-CHAINS = [(60, 10), (60, 11), (60, 14), (60, 22), (60, 23), (55, 10), (55, 14), (55, 15), (55, 16), (55, 29),
+CHAINS = [(60, 10), (60, 11), (60, 12), (60, 13), (60, 14), (60, 22), (60, 23), (55, 10), (55, 14), (55, 15), (55, 16), (55, 29),
           (55, 30), (36, 4)]
 
 

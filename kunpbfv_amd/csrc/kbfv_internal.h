@@ -208,6 +208,11 @@ int kb_ntt(const kbfv_context *c, int dir, const uint64_t *src, uint64_t *dst, i
 // values in [0, 4q), for consumers that fold n^-1 into their first constant
 int kb_intt_noscale(const kbfv_context *c, const uint64_t *src, uint64_t *dst, int mod0, int limbs, int polys,
                     int batch, long sB, long sY, long sL, long dB, long dY, long dL, hipStream_t st);
+// kb_intt_noscale of 2 batch entries, the first half read from src1, the second from
+// src2 (same strides), into consecutive entries of dst
+int kb_intt_noscale_pair(const kbfv_context *c, const uint64_t *src1, const uint64_t *src2, uint64_t *dst, int mod0,
+                         int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
+                         hipStream_t st);
 // contiguous [batch*polys][limbs][N] in place
 int kb_ntt_inplace(const kbfv_context *c, int dir, uint64_t *data, int mod0, int limbs, int polys,
                    hipStream_t st);

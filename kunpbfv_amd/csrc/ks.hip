@@ -245,7 +245,9 @@ __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in
 }  // namespace
 
 bool kb_modup_moddown_fused(const kbfv_context *c) {
-    return c->pn == 1 && ((c->tn == 4 && c->gamma == 2) || (c->tn == 3 && c->gamma == 1));
+    return (c->pn == 1 && ((c->tn == 4 && c->gamma == 2) || (c->tn == 3 && c->gamma == 1) ||
+                           (c->tn == 2 && c->gamma == 1))) ||
+           (c->pn == 2 && c->tn == 4 && c->gamma == 2);
 }
 
 static int modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, const uint64_t *add,
@@ -264,6 +266,10 @@ static int modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *ou
     KB_MUMD(3, 1, 1, false)
     KB_MUMD(4, 2, 1, true)
     KB_MUMD(3, 1, 1, true)
+    KB_MUMD(2, 1, 1, false)
+    KB_MUMD(2, 1, 1, true)
+    KB_MUMD(4, 2, 2, false)
+    KB_MUMD(4, 2, 2, true)
 #undef KB_MUMD
     KB_REQUIRE(!nosc, "unscaled modUp input needs a fused shape");
     // other shapes: the two kernels through the PQ buffer

@@ -48,12 +48,12 @@ __host__ __device__ constexpr bool pass_ok(int log_n, int log_s, int log_t, bool
 }
 __host__ __device__ constexpr int col_log_default(int log_n) { return (log_n + 1) / 2; }
 
-template <int LOG_S, bool COLUMN, int LOG_T>
+template <int LOG_S, bool COLUMN, int LOG_T, int VPT = LOG_R>
 struct Geo {
     static constexpr int TILE = 1 << LOG_T;    // elements per workgroup
     static constexpr int S = 1 << LOG_S;
     static constexpr int C = TILE / S;         // sub-transforms per workgroup
-    static constexpr int T = TILE >> LOG_R;    // threads per workgroup
+    static constexpr int T = TILE >> VPT;      // threads per workgroup
     static constexpr int ROWP = S + S / 16;    // row pass: one pad word per 16
     static constexpr int WORDS = COLUMN ? TILE : C * ROWP;
     __device__ static __forceinline__ int addr(int c, int k) {
@@ -85,11 +85,11 @@ __device__ __forceinline__ void gs_bfly(uint64_t &a, uint64_t &b, kbfv_tw w, uin
 // The twiddles of the one butterfly group thread threadIdx.x takes in a round
 // (rounds with exactly one group per thread), in the order the round consumes
 // them: level j of the round, sub-block m -> slot (1 << j) - 1 + m.
-template <int LR, int LOG_S, bool COLUMN, int LOG_T>
+template <int LR, int LOG_S, bool COLUMN, int LOG_T, int VPT = LOG_R>
 __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, const kbfv_tw *tab,
                                                const int log_n, const int g0, const int grp0,
                                                const int stride) {
-    using G = Geo<LOG_S, COLUMN, LOG_T>;
+    using G = Geo<LOG_S, COLUMN, LOG_T, VPT>;
     constexpr int S = G::S, C = G::C, RR = 1 << LR;
     const int grp = threadIdx.x;
     int c, u;
@@ -123,7 +123,7 @@ __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, con
 // 128-byte runs); it writes them back to the tile or, when GOUT, straight to
 // global memory with the final reduction of the last pass (FIN).
 template <int LR, int LOG_S, bool COLUMN, int LOG_T, bool FWD, bool NINV, bool GIN = false,
-          bool GOUT = false, bool FIN = false, bool PRE = false, bool W1 = false, bool DIG = false>
+          bool GOUT = false, bool FIN = false, bool PRE = false, bool W1 = false, bool DIG = false, int VPT = LOG_R>
 __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const kbfv_tw *tab,
                                           const int log_n, const int g0, const int grp0,
                                           const int stride, const uint64_t q, const kbfv_tw ninv,
@@ -131,7 +131,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                                           uint64_t *__restrict__ gout = nullptr,
                                           const kbfv_tw (*pre)[(1 << LR) - 1] = nullptr,
                                           const int dshift = 0, const uint64_t dmask = ~0ULL) {
-    using G = Geo<LOG_S, COLUMN, LOG_T>;
+    using G = Geo<LOG_S, COLUMN, LOG_T, VPT>;
     constexpr int S = G::S, C = G::C, RR = 1 << LR;
     constexpr int NG = C * (S >> LR);
     const uint64_t q4 = q << 2;
@@ -225,10 +225,10 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
 }
 
 // coalesced global -> LDS copy of the workgroup's tile
-template <int LOG_S, bool COLUMN, int LOG_T>
+template <int LOG_S, bool COLUMN, int LOG_T, int VPT = LOG_R>
 __device__ __forceinline__ void stage_in(uint64_t *tile, const uint64_t *__restrict__ in, int grp0,
                                          int stride) {
-    using G = Geo<LOG_S, COLUMN, LOG_T>;
+    using G = Geo<LOG_S, COLUMN, LOG_T, VPT>;
     constexpr int S = G::S, C = G::C, T = G::T;
 #pragma unroll
     for (int j = 0; j < G::TILE / T; ++j) {
@@ -344,7 +344,8 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     k_ntt_pass(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
                const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
                const kbfv_tw *__restrict__ w1_tab, const uint64_t *__restrict__ mods, int mod0, int limbs,
-               int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL, int xcd) {
+               int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL, int xcd,
+               const uint64_t *__restrict__ src2, int half) {
     using G = Geo<LOG_S, COLUMN, LOG_T>;
     constexpr int groups = (1 << (LOG_N - LOG_S)) / G::C;  // workgroups per limb
     __shared__ uint64_t tile[G::WORDS];
@@ -355,9 +356,96 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     bid /= polys;
     const int bi = bid % batch;
     const int l = bid / batch;
-    pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, src + bi * sB + y * sY + l * sL,
-                                                         dst + bi * dB + y * dY + l * dL, tw, ninv_tab, w1_tab,
-                                                         mods, mod0 + l, grp0);
+    const uint64_t *in = bi < half ? src + bi * sB : src2 + (bi - half) * sB;
+    pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, in + y * sY + l * sL, dst + bi * dB + y * dY + l * dL,
+                                                         tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
+}
+
+// A pass for few transforms (the chip is not full and a wave's own chain of
+// butterflies sets the time): four values per thread and tiles of 2^10 (2^11 where
+// a column row would fall below 64 bytes), so a transform spreads over more waves
+// and CUs; radix-4 rounds (and a radix-2 one for an odd count of levels) whose
+// twiddles are all loaded before the data.
+// Bound by latency: a launch of 16 K to 240 K words takes 8.3 to 11 us for both
+// passes where the tiles of 2^12 (8 values a thread) take 13 to 16; 8 values with
+// the same preload take 10 to 13.
+template <int LOG_S, bool COLUMN>
+struct SmallGeo {
+    static constexpr int VPT = 2;
+    static constexpr int LOG_T = COLUMN && LOG_S == 8 ? 11 : 10;
+    static constexpr int NR = (LOG_S + 1) / 2;
+    static constexpr int lr(int k) { return k == NR - 1 && LOG_S % 2 ? 1 : 2; }
+};
+
+template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE, int K>
+__device__ __forceinline__ void small_twiddles(kbfv_tw (*pre)[3], const kbfv_tw *tab, int g0, int grp0, int stride) {
+    using SG = SmallGeo<LOG_S, COLUMN>;
+    if constexpr (K < SG::NR && SG::lr(K) == 2) {
+        round_twiddles<2, LOG_S, COLUMN, SG::LOG_T, SG::VPT>(pre[K], 2 * K, tab, LOG_N, g0, grp0, stride);
+        small_twiddles<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, K + 1>(pre, tab, g0, grp0, stride);
+    }
+}
+
+// rounds in the transform's order from the K-th on
+template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE, int K>
+__device__ __forceinline__ void small_rounds(uint64_t *tile, const kbfv_tw (*pre)[3], const kbfv_tw *tab, int g0,
+                                             int grp0, int stride, uint64_t q, kbfv_tw ninv, const uint64_t *in,
+                                             uint64_t *out) {
+    using SG = SmallGeo<LOG_S, COLUMN>;
+    if constexpr (K < SG::NR) {
+        constexpr int R = FWD ? K : SG::NR - 1 - K, LR = SG::lr(R);
+        constexpr bool LAST = (FWD != COLUMN), NI = !FWD && LAST && !NOSCALE;
+        // stride-1 rounds of the row pass go through the tile for their global access
+        constexpr bool GIN = K == 0 && (FWD || COLUMN), GOUT = K == SG::NR - 1 && (!FWD || COLUMN);
+        ntt_round<LR, LOG_S, COLUMN, SG::LOG_T, FWD, NI, GIN, GOUT, GOUT && LAST && !NOSCALE, LR == 2, NOSCALE, false,
+                  SG::VPT>(tile, 2 * R, tab, LOG_N, g0, grp0, stride, q, ninv, in, out,
+                           (const kbfv_tw(*)[(1 << LR) - 1]) & pre[R][0]);
+        small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, K + 1>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
+    }
+}
+
+template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE>
+__global__ void __launch_bounds__((1 << SmallGeo<LOG_S, COLUMN>::LOG_T) >> 2)
+    k_ntt_small(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, const kbfv_tw *__restrict__ tw,
+                const kbfv_tw *__restrict__ ninv_tab, const kbfv_tw *__restrict__ w1_tab,
+                const uint64_t *__restrict__ mods, int mod0, int limbs, int polys, int batch, long sB, long sY,
+                long sL, long dB, long dY, long dL, const uint64_t *__restrict__ src2, int half) {
+    using SG = SmallGeo<LOG_S, COLUMN>;
+    using G = Geo<LOG_S, COLUMN, SG::LOG_T, SG::VPT>;
+    constexpr int groups = (1 << (LOG_N - LOG_S)) / G::C, n = 1 << LOG_N, stride = n >> LOG_S;
+    constexpr int g0 = COLUMN ? 0 : LOG_N - LOG_S;
+    constexpr bool LAST = (FWD != COLUMN), NI = !FWD && LAST && !NOSCALE;
+    __shared__ uint64_t tile[G::WORDS];
+    int bid = blockIdx.x;
+    const int grp0 = bid % groups;
+    bid /= groups;
+    const int y = bid % polys;
+    bid /= polys;
+    const int bi = bid % batch;
+    const int l = bid / batch, m = mod0 + l;
+    const uint64_t *in = (bi < half ? src + bi * sB : src2 + (bi - half) * sB) + y * sY + l * sL;
+    uint64_t *out = dst + bi * dB + y * dY + l * dL;
+    const kbfv_tw *tab = tw + ((size_t)m * 2 + (FWD ? 0 : 1)) * n;
+    kbfv_tw pre[SG::NR][3];
+    small_twiddles<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, 0>(pre, tab, g0, grp0, stride);
+    const uint64_t q = mods[m];
+    const kbfv_tw ninv = NI ? ninv_tab[m] : (NOSCALE ? w1_tab[m] : kbfv_tw{0, 0});
+    if constexpr (!FWD && !COLUMN) {
+        stage_in<LOG_S, COLUMN, SG::LOG_T, SG::VPT>(tile, in, grp0, stride);
+        __syncthreads();
+    }
+    small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, 0>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
+    if constexpr (FWD && !COLUMN) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = threadIdx.x + j * G::T, c = e / G::S, k = e % G::S;
+            uint64_t v = tile[G::addr(c, k)];
+            v = kb_csub_sel(v, 0 - (q << 2));
+            v = kb_csub_sel(v, 0 - (q << 1));
+            v = kb_csub_sel(v, 0 - q);
+            out[(grp0 * G::C + c) * G::S + k] = v;
+        }
+    }
 }
 
 // ragged batch: descriptor i = {src, dst, s_limb, d_limb, mod0, limbs} (int64 words),
@@ -400,6 +488,9 @@ struct pass_args {
     long sB, sY, sL, dB, dY, dL;
     int xcd;
     hipStream_t st;
+    // batch entries from `half` on come from src2 (half = batch: one source)
+    const uint64_t *src2 = nullptr;
+    int half = 0x7fffffff;
 };
 
 template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE>
@@ -414,9 +505,43 @@ int launch_pass(const pass_args &a) {
         KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
         hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>), dim3((unsigned)blocks), dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv,
                            a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB, a.dY,
-                           a.dL, a.xcd);
+                           a.dL, a.xcd, a.src2, a.half);
         KB_LAUNCH_CHECK();
         return KBFV_OK;
+    }
+}
+
+template <int LOG_N, bool COLUMN, bool FWD, bool NOSCALE>
+int launch_small(const pass_args &a) {
+    constexpr int LOG_S = COLUMN ? col_log_default(LOG_N) : LOG_N - col_log_default(LOG_N);
+    using SG = SmallGeo<LOG_S, COLUMN>;
+    using G = Geo<LOG_S, COLUMN, SG::LOG_T, SG::VPT>;
+    const long blocks = ((1L << (LOG_N - LOG_S)) / G::C) * a.limbs * a.polys * a.batch;
+    KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
+    hipLaunchKernelGGL((k_ntt_small<LOG_N, LOG_S, COLUMN, FWD, NOSCALE>), dim3((unsigned)blocks), dim3(G::T), 0, a.st,
+                       a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys,
+                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.src2, a.half);
+    KB_LAUNCH_CHECK();
+    return KBFV_OK;
+}
+
+template <int LOG_N>
+int small_transform(int dir, bool noscale, const pass_args &first, const pass_args &second) {
+    if (dir > 0) {
+        KB_TRY((launch_small<LOG_N, true, true, false>(first)));
+        return launch_small<LOG_N, false, true, false>(second);
+    }
+    KB_TRY((launch_small<LOG_N, false, false, false>(first)));
+    return noscale ? launch_small<LOG_N, true, false, true>(second) : launch_small<LOG_N, true, false, false>(second);
+}
+
+int small_transform_n(int log_n, int dir, bool noscale, const pass_args &first, const pass_args &second) {
+    switch (log_n) {
+        case 12: return small_transform<12>(dir, noscale, first, second);
+        case 13: return small_transform<13>(dir, noscale, first, second);
+        case 14: return small_transform<14>(dir, noscale, first, second);
+        case 15: return small_transform<15>(dir, noscale, first, second);
+        default: return small_transform<16>(dir, noscale, first, second);
     }
 }
 
@@ -478,7 +603,7 @@ __global__ void __launch_bounds__((1 << LOG_N) >> LOG_R)
     k_ntt_limb(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, const kbfv_tw *__restrict__ tw,
                const kbfv_tw *__restrict__ ninv_tab, const kbfv_tw *__restrict__ w1_tab,
                const uint64_t *__restrict__ mods, int mod0, int limbs, int polys, int batch, long sB, long sY,
-               long sL, long dB, long dY, long dL, int xcd) {
+               long sL, long dB, long dY, long dL, int xcd, const uint64_t *__restrict__ src2, int half) {
     static_assert(LOG_N >= 12 && LOG_N <= 14, "one limb per workgroup up to 2^14");
     using G = Geo<LOG_N, false, LOG_N>;
     constexpr int T = G::T;
@@ -492,7 +617,7 @@ __global__ void __launch_bounds__((1 << LOG_N) >> LOG_R)
     const int m = mod0 + l;
     const uint64_t q = mods[m];
     const kbfv_tw *tab = tw + ((size_t)m * 2 + (FWD ? 0 : 1)) * n;
-    const uint64_t *in = src + bi * sB + y * sY + l * sL;
+    const uint64_t *in = (bi < half ? src + bi * sB : src2 + (bi - half) * sB) + y * sY + l * sL;
     uint64_t *out = dst + bi * dB + y * dY + l * dL;
     constexpr bool NI = !FWD && !NOSCALE;
     const kbfv_tw ninv = NI ? ninv_tab[m] : (NOSCALE ? w1_tab[m] : kbfv_tw{0, 0});
@@ -603,7 +728,7 @@ int launch_limb(const pass_args &a) {
     KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
     hipLaunchKernelGGL((k_ntt_limb<LOG_N, FWD, NOSCALE>), dim3((unsigned)blocks), dim3((1 << LOG_N) >> LOG_R), 0, a.st,
                        a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys,
-                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd);
+                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd, a.src2, a.half);
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }
@@ -620,12 +745,25 @@ int launch_limb_n(const pass_args &a) {
     }
 }
 
+// Up to this many words a transform under plan 0 takes the small-tile kernels. Both
+// passes together (us, tiles / small tiles): N=2^12 120 rows (480K words) 15.3/12.0,
+// 240 rows 16.9/19.1; N=2^14 30 rows (480K) 15.8/15.0, 60 rows 17.2/23.2; N=2^16 4
+// rows (256K) 16.4/11.7, 8 rows (512K) 15.6/15.0, 15 rows 19.0/22.6. Above it the
+// chip is full of tiles either way and the wider rounds' fewer LDS passes win.
+constexpr long SMALL_WORDS = 1L << 19;
+
 int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, const uint64_t *src, uint64_t *dst,
                   int mod0, int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
-                  hipStream_t st) {
+                  hipStream_t st, const uint64_t *src2 = nullptr) {
     const plan_fields f = decode_plan(c->log_n, plan);
+    const int half = src2 ? batch / 2 : batch;
+    if (plan == 0 && ((long)limbs * polys * batch << c->log_n) <= SMALL_WORDS) {
+        const pass_args first{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, 0, st, src2, half};
+        const pass_args second{c, dst, dst, mod0, limbs, polys, batch, dB, dY, dL, dB, dY, dL, 0, st};
+        return small_transform_n(c->log_n, dir, noscale, first, second);
+    }
     if (single_pass(c->log_n, f)) {
-        const pass_args a{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, f.col_x, st};
+        const pass_args a{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, f.col_x, st, src2, half};
         if (dir > 0) return launch_limb_n<true, false>(a);
         return noscale ? launch_limb_n<false, true>(a) : launch_limb_n<false, false>(a);
     }
@@ -656,6 +794,12 @@ int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, c
         if (cap && dim == 2) cl = kn, cm = mod0 + k0, so = k0 * sL, dof = k0 * dL;
         pass_args first{c, src + so, dst + dof, cm, cl, cp, cb, sB, sY, sL, dB, dY, dL,
                         dir > 0 ? f.col_x : f.row_x, st};
+        if (src2) {  // a chunk over the batch starts at entry k0
+            const bool by_batch = cap && dim == 0;
+            first.src2 = by_batch ? src2 : src2 + so;
+            first.half = std::max(0, half - (by_batch ? k0 : 0));
+            if (by_batch && k0 > half) first.src2 += (k0 - half) * sB;
+        }
         pass_args second{c, dst + dof, dst + dof, cm, cl, cp, cb, dB, dY, dL, dB, dY, dL,
                          dir > 0 ? f.row_x : f.col_x, st};
         if (dir > 0) {
@@ -695,6 +839,15 @@ int kb_intt_noscale(const kbfv_context *c, const uint64_t *src, uint64_t *dst, i
     KB_TRY(check_args(c, src, dst, mod0, limbs, polys, batch));
     const uint32_t plan = plan_for(c, -1, (long)limbs * polys * batch);
     return ntt_with_plan(c, -1, true, plan, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, st);
+}
+
+int kb_intt_noscale_pair(const kbfv_context *c, const uint64_t *src1, const uint64_t *src2, uint64_t *dst, int mod0,
+                         int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
+                         hipStream_t st) {
+    KB_TRY(check_args(c, src1, dst, mod0, limbs, polys, batch));
+    KB_REQUIRE(src2, "null argument");
+    const uint32_t plan = plan_for(c, -1, 2L * limbs * polys * batch);
+    return ntt_with_plan(c, -1, true, plan, src1, dst, mod0, limbs, polys, 2 * batch, sB, sY, sL, dB, dY, dL, st, src2);
 }
 
 namespace {

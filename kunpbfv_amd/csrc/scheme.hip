@@ -280,10 +280,9 @@ int mult_chunk(const kbfv_context *c, const uint64_t *rlk, const uint64_t *ct1, 
     const long CTS = 2 * qn * N;  // ciphertext stride
     // 1. INTT of both inputs (out of place; the NTT-domain inputs stay for the
     // tensor), left N times too large: the base extension folds n^-1 in
-    KB_TRY(kb_intt_noscale(c, ct1, w.X1, c->oQ, qn, 2, cb, CTS, qn * N, N, CTS, qn * N, N, st));
-    KB_TRY(kb_intt_noscale(c, ct2, w.X2, c->oQ, qn, 2, cb, CTS, qn * N, N, CTS, qn * N, N, st));
-    // 2. HPS base extension Q -> R, 3. NTT over R
     // (X2 follows X1 and R2 follows R1: one launch covers both ciphertexts)
+    KB_TRY(kb_intt_noscale_pair(c, ct1, ct2, w.X1, c->oQ, qn, 2, cb, CTS, qn * N, N, CTS, qn * N, N, st));
+    // 2. HPS base extension Q -> R, 3. NTT over R
     KB_TRY(kb_bconv(c, true, w.X1, qn * N, w.R1, rn * N, 4 * cb, st, true));
     KB_TRY(kb_ntt(c, +1, w.R1, w.R1, c->oR, rn, 4 * cb, 1, 0, rn * N, N, 0, rn * N, N, st));
     // 4. tensor over QR, 5. INTT over QR
@@ -680,8 +679,7 @@ extern "C" int kbfv_mult_tensor(const kbfv_context *c, const uint64_t *ct1, cons
         MultWs w;
         mult_layout(c, n, ws, &w);
         const uint64_t *a = ct1 + b0 * CTS, *b = ct2 + b0 * CTS;
-        KB_TRY(kb_intt_noscale(c, a, w.X1, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
-        KB_TRY(kb_intt_noscale(c, b, w.X2, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
+        KB_TRY(kb_intt_noscale_pair(c, a, b, w.X1, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
         KB_TRY(kb_bconv(c, true, w.X1, qn * N, w.R1, rn * N, 4 * n, s, true));
         KB_TRY(kb_ntt(c, +1, w.R1, w.R1, c->oR, rn, 4 * n, 1, 0, rn * N, N, 0, rn * N, N, s));
         KB_TRY(kb_tensor_qr(c, a, b, w.R1, w.R2, w.D3, n, s));
@@ -712,8 +710,7 @@ extern "C" int kbfv_mult_before_ip(const kbfv_context *c, const uint64_t *ct1, c
         mult_layout(c, n, ws, &w);
         const uint64_t *a = ct1 + b0 * CTS, *b = ct2 + b0 * CTS;
         // steps 1-8 of the fused pipeline (mult_chunk), the digits going to ip_in
-        KB_TRY(kb_intt_noscale(c, a, w.X1, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
-        KB_TRY(kb_intt_noscale(c, b, w.X2, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
+        KB_TRY(kb_intt_noscale_pair(c, a, b, w.X1, c->oQ, qn, 2, n, CTS, qn * N, N, CTS, qn * N, N, s));
         KB_TRY(kb_bconv(c, true, w.X1, qn * N, w.R1, rn * N, 4 * n, s, true));
         KB_TRY(kb_ntt(c, +1, w.R1, w.R1, c->oR, rn, 4 * n, 1, 0, rn * N, N, 0, rn * N, N, s));
         KB_TRY(kb_tensor_qr(c, a, b, w.R1, w.R2, w.D3, n, s));

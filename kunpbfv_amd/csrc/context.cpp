@@ -46,6 +46,19 @@ uint64_t powmod(uint64_t a, uint64_t e, uint64_t q) {
 uint64_t invmod(uint64_t a, uint64_t q) { return powmod(a % q, q - 2, q); }
 uint64_t shoup(uint64_t w, uint64_t q) { return (uint64_t)(((kb_u128_host)w << 64) / q); }
 kbfv_tw tw_of(uint64_t w, uint64_t q) { return kbfv_tw{w, shoup(w, q)}; }
+// w as the sum w1 2^28 + w0 of signed halves, w1 and w0 in the high and low word; of
+// w and w - q the one whose w1 is a 32-bit number, the smaller if both are
+uint64_t fold_halves(uint64_t w, uint64_t q) {
+    const int64_t top = (1LL << 59) - (1LL << 27);
+    const int64_t v = (int64_t)w < top && w <= q / 2 ? (int64_t)w : (int64_t)w - (int64_t)q;
+    const int64_t w1 = (v + (1LL << 27)) >> 28, w0 = v - (w1 << 28);
+    return ((uint64_t)(uint32_t)(int32_t)w1 << 32) | (uint32_t)(int32_t)w0;
+}
+// a transform's constant in the form its kernels take for this prime
+kbfv_tw ntt_tw_of(uint64_t w, uint64_t q) {
+    if (!kb_fold_prime(q)) return tw_of(w, q);
+    return kbfv_tw{fold_halves(w, q), fold_halves((uint64_t)(((kb_u128_host)w << 32) % q), q)};
+}
 
 bool is_prime(uint64_t n) {
     static const uint64_t bases[12] = {2, 3, 5, 7, 11, 13, 17, 19, 23, 29, 31, 37};
@@ -631,11 +644,11 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
             f[nx] = mulmod(psi, f[pr], qm);
             iv[nx] = mulmod(psiinv, iv[pr], qm);
         }
-        inv_w1[m] = tw_of(iv[1], qm);  // the last inverse stage's twiddle without n^-1
+        inv_w1[m] = ntt_tw_of(iv[1], qm);  // the last inverse stage's twiddle without n^-1
         iv[1] = mulmod(iv[1], ni, qm);
         kbfv_tw *base = tw.data() + (size_t)m * 2 * N;
-        for (int i = 0; i < N; i++) base[i] = tw_of(f[i], qm), base[N + i] = tw_of(iv[i], qm);
-        ninv[m] = tw_of(ni, qm);
+        for (int i = 0; i < N; i++) base[i] = ntt_tw_of(f[i], qm), base[N + i] = ntt_tw_of(iv[i], qm);
+        ninv[m] = ntt_tw_of(ni, qm);
     }
     std::vector<uint64_t> mu(2 * c->nmod);
     for (int m = 0; m < c->nmod; m++) {

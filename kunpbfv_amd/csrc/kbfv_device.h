@@ -179,6 +179,45 @@ __device__ __forceinline__ void kb_mad(int64_t &acc, int a, int b) {
     acc = (int64_t)((uint64_t)acc + (uint64_t)((int64_t)a * b));
 }
 __device__ __forceinline__ void kb_mad(uint64_t &acc, uint32_t a, uint32_t b) { acc += (uint64_t)a * b; }
+// Multiplication modulo a prime q = 2^60 - c, 0 < c <= 2^26, on signed values.  x =
+// x1 2^32 + x0 with x0 signed; the constant w (twiddle) and w' = w 2^32 mod q are
+// split at 28 bits into signed 32-bit halves, w = w1 2^28 + w0.  Then
+// x w = x0 w + x1 w' = A + 2^28 B, A = x0 w0 + x1 w'0, B = x0 w1 + x1 w'1, and with
+// B = v 2^32 + b, 0 <= b < 2^32, the part v 2^60 is v c modulo q: A + 2^28 b + v c.
+// Six multiply-adds with no carry between them.  |w|, |w'| <= 2^59 and |w0|, |w'0| <=
+// 2^27, so for |x| < 8 (2^60 - 2^32) B stays below 2^63 and for |x| <= X 2^60 the result
+// lies between -d 2^60 and (1 + d) 2^60, d = (1/4 + X/32) (1 + c 2^-28).
+__host__ __device__ __forceinline__ bool kb_fold_prime(uint64_t q) { return (q >> 26) == (1ULL << 34) - 1; }
+__device__ __forceinline__ uint32_t kb_fold_c(uint64_t q) { return (uint32_t)((1ULL << 60) - q); }
+// x w + add, w as a pair of packed halves (w0 | w1 << 32); k28 = 2^28
+__device__ __forceinline__ uint64_t kb_fmul(uint64_t x, kbfv_tw w, uint32_t c, uint32_t k28, uint64_t add) {
+    const int x0 = (int)(uint32_t)x, x1 = (int)(uint32_t)((x + (1ULL << 31)) >> 32);
+    int64_t A = (int64_t)add, B = 0;
+    kb_mad(B, x0, (int)(uint32_t)(w.w >> 32));
+    kb_mad(A, x0, (int)(uint32_t)w.w);
+    kb_mad(B, x1, (int)(uint32_t)(w.ws >> 32));
+    kb_mad(A, x1, (int)(uint32_t)w.ws);
+    uint64_t r = kb_mad32((uint32_t)B, k28, (uint64_t)A);
+    int64_t s = (int64_t)r;
+    kb_mad(s, (int)(uint32_t)((uint64_t)B >> 32), (int)c);
+    return (uint64_t)s;
+}
+// signed x -> x mod q up to [-8c, 2^60 + 7c]
+__device__ __forceinline__ uint64_t kb_sfold(uint64_t x, uint32_t c) {
+    const uint32_t hi = (uint32_t)(x >> 32);
+    int64_t r = (int64_t)(((uint64_t)(hi & 0x0fffffffu) << 32) | (uint32_t)x);
+    kb_mad(r, (int)hi >> 28, (int)c);
+    return (uint64_t)r;
+}
+// any 64-bit x -> x mod q up to [0, 2^60 + 15c]
+__device__ __forceinline__ uint64_t kb_ufold(uint64_t x, uint32_t c) {
+    const uint32_t hi = (uint32_t)(x >> 32);
+    return kb_mad32(hi >> 28, c, ((uint64_t)(hi & 0x0fffffffu) << 32) | (uint32_t)x);
+}
+// signed x, |x| <= 7.9 2^60 -> [0, q)
+__device__ __forceinline__ uint64_t kb_fold_canon(uint64_t x, uint64_t q, uint64_t nq, uint32_t c) {
+    return kb_csub_sel(kb_ufold(x + (q << 3), c), nq);
+}
 // Marks a 32-bit register value as changed.  A multiplicand that a loop reads in
 // every pass is otherwise widened to 64 bits ahead of the loop and takes a
 // register pair for its whole length.

@@ -72,8 +72,10 @@ struct kb_conv_in {
 struct kb_dev_tables {
     const uint64_t *mod;   // [nmod]
     const uint64_t *mu;    // [nmod][2] Barrett floor(2^128/q): lo, hi
-    const kbfv_tw *tw;     // [nmod][2][N]: forward psi table, inverse psi table (bit-reversed)
-    const kbfv_tw *ninv;   // [nmod] n^-1 with Shoup companion
+    // [nmod][2][N]: forward psi table, inverse psi table (bit-reversed); like ninv and inv_w1
+    // value and Shoup companion, or kb_fmul halves where kb_fold_prime(modulus)
+    const kbfv_tw *tw;
+    const kbfv_tw *ninv;   // [nmod] n^-1
 
     // HPS base conversion Q -> R and R -> Q
     const kbfv_tw *q_hatinv;       // [qn]

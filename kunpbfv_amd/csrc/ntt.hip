@@ -12,14 +12,20 @@
 //   column pass  -- C adjacent columns of stride N/N1 (coalesced C*8-byte rows),
 //                   global stages 0 .. log2(N1)-1
 //   row pass     -- C contiguous chunks of N2 elements, remaining stages
-// Forward = column then row; inverse = row then column.  Values stay lazy in
+// Forward = column then row; inverse = row then column.  Butterflies modulo primes
+// 2^60 - c (c <= 2^26, the chains of 60-bit primes) work on signed values with ten
+// instructions and no conditional subtraction; a register round folds its values
+// back to 60 bits.  Modulo other primes values stay lazy in
 // [0, 8q) (forward) / [0, 4q) (inverse) between stages (moduli are below 2^60,
-// so every sum stays below 2^63) and are reduced once on the final store.  The
-// twiddle products use an under-estimated Shoup quotient (one 32-bit high
-// product and two carries fewer, result in [0, 4q)), and conditional
-// subtractions select on the sign word with v_bfi_b32, so no carry or compare
-// result passes through an SGPR.  Twiddles are (w, Shoup w') pairs read as one 16-byte load,
-// one load per distinct twiddle per thread.  The grid is ordered limb-slowest so
+// so every sum stays below 2^63); the twiddle products use an under-estimated
+// Shoup quotient (one 32-bit high product and two carries fewer, result in [0, 4q)),
+// and conditional subtractions select on the sign word with v_bfi_b32, so no
+// carry or compare result passes through an SGPR.  Either way values are reduced
+// once on the final store.  A radix-16 round takes 600 instructions in the first
+// form and 970 in the second; both passes of 256 x 8 limbs at N=2^14, forward: 233 us
+// against 268, of 480 rows at N=2^14: 59 against 69, of 120 rows at N=2^16: 65 against
+// 75 (from there on HBM bounds them at 3.8 TB/s).  Twiddles are 16 bytes, read in one
+// load per distinct twiddle per thread.  The grid is ordered limb-slowest so
 // that every workgroup in flight shares one modulus' tables in L2.
 //
 // Plans: the split point (column pass length 2^LOG_S, the row pass takes the
@@ -82,6 +88,40 @@ __device__ __forceinline__ void gs_bfly(uint64_t &a, uint64_t &b, kbfv_tw w, uin
     b = v;
 }
 
+// Butterflies for primes 2^60 - c, c < 2^26: values are signed, twiddles signed
+// halves (kb_fmul).  The product comes on top of its addend, so the sum is free and
+// the difference is 2a - (a + t); six multiply-adds in place of the Shoup product's
+// ten multiplies, and no conditional subtraction.  With c <= 2^26 a product of |x| <= X 2^60 lies
+// in (-d, 1 + d) 2^60, d = 1.25 (1/4 + X/32).  Forward: [0, 1] grows to (-5.8, 6.8)
+// over four levels.  Inverse: values in (-0.9, 1.9) give sums below 7.6 over two
+// levels, the sums are folded back to [0, 1] there, products stay in (-0.6, 1.6).
+__device__ __forceinline__ void ct_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
+    const uint64_t s = kb_fmul(b, w, c, k28, a);
+    b = (a << 1) - s;
+    a = s;
+}
+
+template <bool RED>
+__device__ __forceinline__ void gs_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
+    const uint64_t u = a + b;
+    b = kb_fmul(a - b, w, c, k28, 0);
+    a = RED ? kb_sfold(u, c) : u;
+}
+
+// ntt_round's options
+enum : int {
+    RD_NINV = 1,   // n^-1 multiply at stage 0
+    RD_GIN = 2,    // values straight from global memory
+    RD_GOUT = 4,   // values straight to global memory
+    RD_FIN = 8,    // ... reduced to [0, q)
+    RD_PRE = 16,   // the twiddles are in `pre`
+    RD_W1 = 32,    // stage 0 takes the unscaled entry 1, passed in ninv
+    RD_DIG = 64,   // the input is one base-2^w digit of the loaded word
+    RD_FOLD = 128, // prime near 2^60: signed values
+    RD_IN = 256,   // first round of the transform (any 64-bit input)
+    RD_OPEN = 512, // RD_FOLD forward: the next reader folds the values
+};
+
 // The twiddles of the one butterfly group thread threadIdx.x takes in a round
 // (rounds with exactly one group per thread), in the order the round consumes
 // them: level j of the round, sub-block m -> slot (1 << j) - 1 + m.
@@ -122,8 +162,7 @@ __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, con
 // (the rounds whose lanes cover adjacent columns / 16 adjacent elements, i.e.
 // 128-byte runs); it writes them back to the tile or, when GOUT, straight to
 // global memory with the final reduction of the last pass (FIN).
-template <int LR, int LOG_S, bool COLUMN, int LOG_T, bool FWD, bool NINV, bool GIN = false,
-          bool GOUT = false, bool FIN = false, bool PRE = false, bool W1 = false, bool DIG = false, int VPT = LOG_R>
+template <int LR, int LOG_S, bool COLUMN, int LOG_T, bool FWD, int FL, int VPT = LOG_R>
 __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const kbfv_tw *tab,
                                           const int log_n, const int g0, const int grp0,
                                           const int stride, const uint64_t q, const kbfv_tw ninv,
@@ -131,6 +170,8 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                                           uint64_t *__restrict__ gout = nullptr,
                                           const kbfv_tw (*pre)[(1 << LR) - 1] = nullptr,
                                           const int dshift = 0, const uint64_t dmask = ~0ULL) {
+    constexpr bool NINV = FL & RD_NINV, GIN = FL & RD_GIN, GOUT = FL & RD_GOUT, FIN = FL & RD_FIN, PRE = FL & RD_PRE,
+                   W1 = FL & RD_W1, DIG = FL & RD_DIG, FOLD = FL & RD_FOLD;
     using G = Geo<LOG_S, COLUMN, LOG_T, VPT>;
     constexpr int S = G::S, C = G::C, RR = 1 << LR;
     constexpr int NG = C * (S >> LR);
@@ -139,6 +180,9 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
     // opaque to the optimizer, which would otherwise turn x + (2^64 - m) back
     // into a subtraction with its carry through an SGPR
     asm volatile("" : "+s"(nq), "+s"(nq4));
+    const uint32_t c60 = kb_fold_c(q);
+    uint32_t k28 = 1u << 28;
+    asm volatile("" : "+s"(k28));  // a multiplier, not a shift and an add
     const int Bs = S >> lam0;
     const int d = Bs >> LR;
     for (int grp = threadIdx.x; grp < NG; grp += G::T) {
@@ -163,6 +207,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                 if constexpr (DIG) x[i] = (x[i] >> dshift) & dmask;
             } else
                 x[i] = tile[G::addr(c, kbase + i * d)];
+            if constexpr (FOLD && (FL & RD_IN)) x[i] = kb_ufold(x[i], c60);
         }
         if constexpr (FWD) {
 #pragma unroll
@@ -179,7 +224,17 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     else
                         w = tab[(1 << gst) + (pos >> (log_n - gst))];
 #pragma unroll
-                    for (int i = i0; i < i0 + h; ++i) ct_bfly(x[i], x[i + h], w, nq, q4, nq4);
+                    for (int i = i0; i < i0 + h; ++i) {
+                        if constexpr (FOLD)
+                            ct_fold(x[i], x[i + h], w, c60, k28);
+                        else
+                            ct_bfly(x[i], x[i + h], w, nq, q4, nq4);
+                    }
+                }
+                if constexpr (FOLD && LR > 4) {
+                    if (j == 3)
+#pragma unroll
+                        for (int i = 0; i < RR; ++i) x[i] = kb_sfold(x[i], c60);
                 }
             }
         } else {
@@ -200,17 +255,30 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     if (W1 && gst == 0) w = ninv;
 #pragma unroll
                     for (int i = i0; i < i0 + h; ++i) {
-                        gs_bfly(x[i], x[i + h], w, nq, q4, nq4);
-                        if (NINV && gst == 0) x[i] = kb_shoup4(x[i], ninv.w, ninv.ws, nq);
+                        if constexpr (FOLD) {
+                            const bool last = GOUT && j == 0;  // folded with the store
+                            if (((LR - j) % 2 == 0 || j == 0) && !last)
+                                gs_fold<true>(x[i], x[i + h], w, c60, k28);
+                            else
+                                gs_fold<false>(x[i], x[i + h], w, c60, k28);
+                            if (NINV && gst == 0) x[i] = kb_fmul(x[i], ninv, c60, k28, 0);
+                        } else {
+                            gs_bfly(x[i], x[i + h], w, nq, q4, nq4);
+                            if (NINV && gst == 0) x[i] = kb_shoup4(x[i], ninv.w, ninv.ws, nq);
+                        }
                     }
                 }
             }
         }
 #pragma unroll
         for (int i = 0; i < RR; ++i) {
+            if constexpr (FOLD && FWD && !FIN && !(FL & RD_OPEN)) x[i] = kb_sfold(x[i], c60);
             if constexpr (GOUT) {
                 uint64_t v = x[i];
-                if constexpr (FIN) {
+                if constexpr (FOLD) {
+                    if constexpr (!FWD) v = FIN || W1 ? kb_ufold(v + (q << 3), c60) : kb_sfold(v, c60);
+                    if constexpr (FIN) v = FWD ? kb_fold_canon(v, q, nq, c60) : kb_csub_sel(v, nq);
+                } else if constexpr (FIN) {
                     if constexpr (FWD) v = kb_csub_sel(v, nq4);
                     v = kb_csub_sel(v, 0 - (q << 1));
                     v = kb_csub_sel(v, nq);
@@ -246,10 +314,19 @@ __device__ __forceinline__ void stage_in(uint64_t *tile, const uint64_t *__restr
     }
 }
 
+// the forward transform's last values, [0, 8q) or signed, to [0, q)
+template <bool FOLD>
+__device__ __forceinline__ uint64_t forward_canon(uint64_t v, uint64_t q) {
+    if constexpr (FOLD) return kb_fold_canon(v, q, 0 - q, kb_fold_c(q));
+    v = kb_csub_sel(v, 0 - (q << 2));
+    v = kb_csub_sel(v, 0 - (q << 1));
+    return kb_csub_sel(v, 0 - q);
+}
+
 // one workgroup's tile of one limb: `in` / `out` address the limb, m is its modulus
 // DIG (forward column pass only): the input value is (word >> dshift) & dmask
-template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool DIG = false>
-__device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__restrict__ in,
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool DIG, bool FOLD>
+__device__ __forceinline__ void pass_tile(uint64_t *tile, const uint64_t *__restrict__ in,
                                           uint64_t *__restrict__ out, const kbfv_tw *__restrict__ tw,
                                           const kbfv_tw *__restrict__ ninv_tab, const kbfv_tw *__restrict__ w1_tab,
                                           const uint64_t *__restrict__ mods, const int m, const int grp0,
@@ -276,20 +353,21 @@ __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__rest
     // the forward pass's first register round (stride S/16) and the inverse pass's last
     // touch 128-byte runs in both layouts; the stride-1 rounds of the row pass
     // go through the LDS tile for both their global load and store.
+    constexpr int FD = FOLD ? RD_FOLD : 0, N1 = FD | (NI ? RD_NINV : 0), FIRST = (FWD == COLUMN) ? RD_IN : 0;
     if constexpr (FWD) {
-        ntt_round<LR0, LOG_S, COLUMN, LOG_T, true, false, true, false, false, false, false, DIG>(
+        ntt_round<LR0, LOG_S, COLUMN, LOG_T, true, FD | FIRST | RD_GIN | (DIG ? RD_DIG : 0)>(
             tile, 0, tab, log_n, g0, grp0, stride, q, ninv, in, nullptr, nullptr, dshift, dmask);
         if constexpr (COLUMN) {
-            ntt_round<LR1, LOG_S, COLUMN, LOG_T, true, false, false, true, LAST>(tile, LR0, tab, log_n, g0, grp0,
-                                                                                 stride, q, ninv, nullptr, out);
+            ntt_round<LR1, LOG_S, COLUMN, LOG_T, true, FD | RD_GOUT>(tile, LR0, tab, log_n, g0, grp0, stride, q, ninv,
+                                                                     nullptr, out);
             return;
         } else {
-            ntt_round<LR1, LOG_S, COLUMN, LOG_T, true, false>(tile, LR0, tab, log_n, g0, grp0, stride, q, ninv);
+            ntt_round<LR1, LOG_S, COLUMN, LOG_T, true, FD | RD_OPEN>(tile, LR0, tab, log_n, g0, grp0, stride, q, ninv);
         }
     } else {
         if constexpr (COLUMN) {
-            ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, NI, true>(tile, LR0, tab, log_n, g0, grp0, stride, q,
-                                                                  ninv, in);
+            ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, N1 | RD_GIN>(tile, LR0, tab, log_n, g0, grp0, stride, q, ninv,
+                                                                     in);
         } else {
             // one butterfly group per thread (a radix-16 round): its twiddles are
             // loaded with the tile, ahead of the barrier, rather than after it
@@ -302,15 +380,17 @@ __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__rest
 #pragma unroll
                 for (int i = 0; i < (1 << LR1) - 1; ++i) asm volatile("" : "+v"(pre[i].w), "+v"(pre[i].ws));
                 __syncthreads();
-                ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, NI, false, false, false, true>(
-                    tile, LR0, tab, log_n, g0, grp0, stride, q, ninv, nullptr, nullptr, &pre);
+                ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, N1 | FIRST | RD_PRE>(tile, LR0, tab, log_n, g0, grp0,
+                                                                                 stride, q, ninv, nullptr, nullptr, &pre);
             } else {
                 stage_in<LOG_S, COLUMN, LOG_T>(tile, in, grp0, stride);
                 __syncthreads();
-                ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, NI>(tile, LR0, tab, log_n, g0, grp0, stride, q, ninv);
+                ntt_round<LR1, LOG_S, COLUMN, LOG_T, false, N1 | FIRST>(tile, LR0, tab, log_n, g0, grp0, stride, q,
+                                                                        ninv);
             }
         }
-        ntt_round<LR0, LOG_S, COLUMN, LOG_T, false, NI, false, true, LAST && !NOSCALE, false, NOSCALE>(
+        ntt_round<LR0, LOG_S, COLUMN, LOG_T, false,
+                  N1 | RD_GOUT | (LAST && !NOSCALE ? RD_FIN : 0) | (NOSCALE ? RD_W1 : 0)>(
             tile, 0, tab, log_n, g0, grp0, stride, q, ninv, nullptr, out);
         return;
     }
@@ -320,14 +400,22 @@ __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__rest
     for (int j = 0; j < G::TILE / T; ++j) {
         const int e = threadIdx.x + j * T;
         const int c = e / S, k = e % S;
-        uint64_t v = tile[G::addr(c, k)];
-        if constexpr (LAST) {
-            v = kb_csub_sel(v, 0 - (q << 2));
-            v = kb_csub_sel(v, 0 - (q << 1));
-            v = kb_csub_sel(v, 0 - q);
-        }
-        out[(grp0 * C + c) * S + k] = v;
+        out[(grp0 * C + c) * S + k] = forward_canon<FOLD>(tile[G::addr(c, k)], q);
     }
+}
+
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool DIG = false>
+__device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
+                                          const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
+                                          const kbfv_tw *__restrict__ w1_tab, const uint64_t *__restrict__ mods,
+                                          const int m, const int grp0, const int dshift = 0,
+                                          const uint64_t dmask = ~0ULL) {
+    if (kb_fold_prime(mods[m]))  // uniform: one modulus per workgroup
+        pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, DIG, true>(tile, in, out, tw, ninv_tab, w1_tab, mods, m,
+                                                                        grp0, dshift, dmask);
+    else
+        pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, DIG, false>(tile, in, out, tw, ninv_tab, w1_tab, mods, m,
+                                                                         grp0, dshift, dmask);
 }
 
 // XCD-aware order: workgroup b runs on XCD b % 8, so when the grid is a
@@ -387,7 +475,7 @@ __device__ __forceinline__ void small_twiddles(kbfv_tw (*pre)[3], const kbfv_tw 
 }
 
 // rounds in the transform's order from the K-th on
-template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE, int K>
+template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE, bool FOLD, int K>
 __device__ __forceinline__ void small_rounds(uint64_t *tile, const kbfv_tw (*pre)[3], const kbfv_tw *tab, int g0,
                                              int grp0, int stride, uint64_t q, kbfv_tw ninv, const uint64_t *in,
                                              uint64_t *out) {
@@ -397,10 +485,17 @@ __device__ __forceinline__ void small_rounds(uint64_t *tile, const kbfv_tw (*pre
         constexpr bool LAST = (FWD != COLUMN), NI = !FWD && LAST && !NOSCALE;
         // stride-1 rounds of the row pass go through the tile for their global access
         constexpr bool GIN = K == 0 && (FWD || COLUMN), GOUT = K == SG::NR - 1 && (!FWD || COLUMN);
-        ntt_round<LR, LOG_S, COLUMN, SG::LOG_T, FWD, NI, GIN, GOUT, GOUT && LAST && !NOSCALE, LR == 2, NOSCALE, false,
+        // folded forward values: every second round and before global memory
+        constexpr bool OPEN = K % 2 == 0 && !GOUT;
+        ntt_round<LR, LOG_S, COLUMN, SG::LOG_T, FWD,
+                  (NI ? RD_NINV : 0) | (GIN ? RD_GIN : 0) | (GOUT ? RD_GOUT : 0) |
+                      (GOUT && LAST && !NOSCALE ? RD_FIN : 0) | (LR == 2 ? RD_PRE : 0) | (NOSCALE ? RD_W1 : 0) |
+                      (FOLD ? RD_FOLD : 0) | (FWD == COLUMN && K == 0 ? RD_IN : 0) |
+                      (OPEN || (K == SG::NR - 1 && !GOUT) ? RD_OPEN : 0),
                   SG::VPT>(tile, 2 * R, tab, LOG_N, g0, grp0, stride, q, ninv, in, out,
                            (const kbfv_tw(*)[(1 << LR) - 1]) & pre[R][0]);
-        small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, K + 1>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
+        small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, FOLD, K + 1>(tile, pre, tab, g0, grp0, stride, q, ninv, in,
+                                                                      out);
     }
 }
 
@@ -434,18 +529,21 @@ __global__ void __launch_bounds__((1 << SmallGeo<LOG_S, COLUMN>::LOG_T) >> 2)
         stage_in<LOG_S, COLUMN, SG::LOG_T, SG::VPT>(tile, in, grp0, stride);
         __syncthreads();
     }
-    small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, 0>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
-    if constexpr (FWD && !COLUMN) {
+    const auto run = [&](auto fold) {
+        constexpr bool FOLD = decltype(fold)::value;
+        small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, FOLD, 0>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
+        if constexpr (FWD && !COLUMN) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int e = threadIdx.x + j * G::T, c = e / G::S, k = e % G::S;
-            uint64_t v = tile[G::addr(c, k)];
-            v = kb_csub_sel(v, 0 - (q << 2));
-            v = kb_csub_sel(v, 0 - (q << 1));
-            v = kb_csub_sel(v, 0 - q);
-            out[(grp0 * G::C + c) * G::S + k] = v;
+            for (int j = 0; j < 4; ++j) {
+                const int e = threadIdx.x + j * G::T, c = e / G::S, k = e % G::S;
+                out[(grp0 * G::C + c) * G::S + k] = forward_canon<FOLD>(tile[G::addr(c, k)], q);
+            }
         }
-    }
+    };
+    if (kb_fold_prime(q))  // uniform
+        run(std::true_type{});
+    else
+        run(std::false_type{});
 }
 
 // ragged batch: descriptor i = {src, dst, s_limb, d_limb, mod0, limbs} (int64 words),
@@ -587,14 +685,17 @@ __host__ __device__ constexpr int limb_round_lam(int log_n, int k) {
     return k == 0 ? 0 : limb_round_lam(log_n, k - 1) + limb_round_log(log_n, k - 1);
 }
 
-template <int LOG_N, int K, bool FWD, bool NI>
+template <int LOG_N, int K, bool FWD, bool NI, bool FOLD>
 __device__ __forceinline__ void limb_rounds_mid(uint64_t *tile, const kbfv_tw *tab, uint64_t q, kbfv_tw ninv) {
     // rounds 1 .. limb_rounds - 1, LDS to LDS: ascending (forward) / descending (inverse)
     if constexpr (K >= 1 && K < limb_rounds(LOG_N)) {
         constexpr int KK = FWD ? K : limb_rounds(LOG_N) - K;
-        ntt_round<limb_round_log(LOG_N, KK), LOG_N, false, LOG_N, FWD, NI>(tile, limb_round_lam(LOG_N, KK), tab,
-                                                                         LOG_N, 0, 0, 1, q, ninv);
-        limb_rounds_mid<LOG_N, K + 1, FWD, NI>(tile, tab, q, ninv);
+        // the forward transform's last values are folded by the store
+        constexpr int FL = (NI ? RD_NINV : 0) | (FOLD ? RD_FOLD : 0) | (!FWD && K == 1 ? RD_IN : 0) |
+                           (FWD && K == limb_rounds(LOG_N) - 1 ? RD_OPEN : 0);
+        ntt_round<limb_round_log(LOG_N, KK), LOG_N, false, LOG_N, FWD, FL>(tile, limb_round_lam(LOG_N, KK), tab, LOG_N,
+                                                                           0, 0, 1, q, ninv);
+        limb_rounds_mid<LOG_N, K + 1, FWD, NI, FOLD>(tile, tab, q, ninv);
     }
 }
 
@@ -621,26 +722,31 @@ __global__ void __launch_bounds__((1 << LOG_N) >> LOG_R)
     uint64_t *out = dst + bi * dB + y * dY + l * dL;
     constexpr bool NI = !FWD && !NOSCALE;
     const kbfv_tw ninv = NI ? ninv_tab[m] : (NOSCALE ? w1_tab[m] : kbfv_tw{0, 0});
-    if constexpr (FWD) {
-        // the radix-16 round of stride N/16 reads global memory in 128-byte runs
-        ntt_round<4, LOG_N, false, LOG_N, true, false, true>(tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, in);
-        limb_rounds_mid<LOG_N, 1, true, false>(tile, tab, q, ninv);
+    const auto run = [&](auto fold) {
+        constexpr bool FOLD = decltype(fold)::value;
+        constexpr int FD = FOLD ? RD_FOLD : 0;
+        if constexpr (FWD) {
+            // the radix-16 round of stride N/16 reads global memory in 128-byte runs
+            ntt_round<4, LOG_N, false, LOG_N, true, FD | RD_GIN | RD_IN>(tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, in);
+            limb_rounds_mid<LOG_N, 1, true, false, FOLD>(tile, tab, q, ninv);
 #pragma unroll
-        for (int j = 0; j < n / T; ++j) {
-            const int k = threadIdx.x + j * T;
-            uint64_t v = tile[G::addr(0, k)];
-            v = kb_csub_sel(v, 0 - (q << 2));
-            v = kb_csub_sel(v, 0 - (q << 1));
-            v = kb_csub_sel(v, 0 - q);
-            out[k] = v;
+            for (int j = 0; j < n / T; ++j) {
+                const int k = threadIdx.x + j * T;
+                out[k] = forward_canon<FOLD>(tile[G::addr(0, k)], q);
+            }
+        } else {
+            stage_in<LOG_N, false, LOG_N>(tile, in, 0, 1);
+            __syncthreads();
+            limb_rounds_mid<LOG_N, 1, false, NI, FOLD>(tile, tab, q, ninv);
+            ntt_round<4, LOG_N, false, LOG_N, false,
+                      FD | (NI ? RD_NINV : 0) | RD_GOUT | (NOSCALE ? RD_W1 : RD_FIN)>(tile, 0, tab, LOG_N, 0, 0, 1, q,
+                                                                                     ninv, nullptr, out);
         }
-    } else {
-        stage_in<LOG_N, false, LOG_N>(tile, in, 0, 1);
-        __syncthreads();
-        limb_rounds_mid<LOG_N, 1, false, NI>(tile, tab, q, ninv);
-        ntt_round<4, LOG_N, false, LOG_N, false, NI, false, true, !NOSCALE, false, NOSCALE>(
-            tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, nullptr, out);
-    }
+    };
+    if (kb_fold_prime(q))  // uniform
+        run(std::true_type{});
+    else
+        run(std::false_type{});
 }
 
 // forward column pass of the external product's digit polynomials, the digit

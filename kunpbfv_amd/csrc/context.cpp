@@ -647,7 +647,11 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
         inv_w1[m] = ntt_tw_of(iv[1], qm);  // the last inverse stage's twiddle without n^-1
         iv[1] = mulmod(iv[1], ni, qm);
         kbfv_tw *base = tw.data() + (size_t)m * 2 * N;
-        for (int i = 0; i < N; i++) base[i] = ntt_tw_of(f[i], qm), base[N + i] = ntt_tw_of(iv[i], qm);
+        for (int i = 0, g = 0; i < N; i++) {
+            if (i >= 2 << g) g++;
+            const int k = i < 1 ? 0 : kb_tw_index(log_n, g, i - (1 << g));
+            base[k] = ntt_tw_of(f[i], qm), base[N + k] = ntt_tw_of(iv[i], qm);
+        }
         ninv[m] = ntt_tw_of(ni, qm);
     }
     std::vector<uint64_t> mu(2 * c->nmod);

@@ -218,6 +218,33 @@ __device__ __forceinline__ uint64_t kb_ufold(uint64_t x, uint32_t c) {
 __device__ __forceinline__ uint64_t kb_fold_canon(uint64_t x, uint64_t q, uint64_t nq, uint32_t c) {
     return kb_csub_sel(kb_ufold(x + (q << 3), c), nq);
 }
+// Butterflies for primes 2^60 - c, c < 2^26: values are signed, twiddles signed
+// halves (kb_fmul).  The product comes on top of its addend, so the sum is free and
+// the difference is 2a - (a + t); six multiply-adds in place of the Shoup product's
+// ten multiplies, and no conditional subtraction.  With c <= 2^26 a product of |x| <= X 2^60 lies
+// in (-d, 1 + d) 2^60, d = 1.25 (1/4 + X/32).  Forward: [0, 1] grows to (-5.8, 6.8)
+// over four levels.  Inverse: values in (-0.9, 1.9) give sums below 7.6 over two
+// levels, the sums are folded back to [0, 1] there, products stay in (-0.6, 1.6).
+__device__ __forceinline__ void ct_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
+    const uint64_t s = kb_fmul(b, w, c, k28, a);
+    b = (a << 1) - s;
+    a = s;
+}
+
+template <bool RED>
+__device__ __forceinline__ void gs_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
+    const uint64_t u = a + b;
+    b = kb_fmul(a - b, w, c, k28, 0);
+    a = RED ? kb_sfold(u, c) : u;
+}
+
+// Place in a limb's twiddle table of group x of level g (2^g groups): levels follow each
+// other; the last five store the groups of one 32-element block 2^(log_n - 5) apart, so
+// that lanes of consecutive blocks read consecutive twiddles.
+__host__ __device__ __forceinline__ int kb_tw_index(int log_n, int g, int x) {
+    const int j = g - (log_n - 5);
+    return (1 << g) + (j <= 0 ? x : ((x & ((1 << j) - 1)) << (log_n - 5)) + (x >> j));
+}
 // Marks a 32-bit register value as changed.  A multiplicand that a loop reads in
 // every pass is otherwise widened to 64 bits ahead of the loop and takes a
 // register pair for its whole length.

@@ -72,7 +72,7 @@ struct kb_conv_in {
 struct kb_dev_tables {
     const uint64_t *mod;   // [nmod]
     const uint64_t *mu;    // [nmod][2] Barrett floor(2^128/q): lo, hi
-    // [nmod][2][N]: forward psi table, inverse psi table (bit-reversed); like ninv and inv_w1
+    // [nmod][2][N]: forward psi table, inverse psi table (kb_tw_index order); like ninv and inv_w1
     // value and Shoup companion, or kb_fmul halves where kb_fold_prime(modulus)
     const kbfv_tw *tw;
     const kbfv_tw *ninv;   // [nmod] n^-1
@@ -215,6 +215,10 @@ int kb_intt_noscale(const kbfv_context *c, const uint64_t *src, uint64_t *dst, i
 int kb_intt_noscale_pair(const kbfv_context *c, const uint64_t *src1, const uint64_t *src2, uint64_t *dst, int mod0,
                          int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
                          hipStream_t st);
+// one-pass transform, every modulus near 2^60; entries from `half` on come from src2
+int kb_ntt_reg(const kbfv_context *c, int dir, bool noscale, const uint64_t *src, uint64_t *dst, int mod0, int limbs,
+               int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL, hipStream_t st,
+               const uint64_t *src2, int half);
 // contiguous [batch*polys][limbs][N] in place
 int kb_ntt_inplace(const kbfv_context *c, int dir, uint64_t *data, int mod0, int limbs, int polys,
                    hipStream_t st);

@@ -88,26 +88,6 @@ __device__ __forceinline__ void gs_bfly(uint64_t &a, uint64_t &b, kbfv_tw w, uin
     b = v;
 }
 
-// Butterflies for primes 2^60 - c, c < 2^26: values are signed, twiddles signed
-// halves (kb_fmul).  The product comes on top of its addend, so the sum is free and
-// the difference is 2a - (a + t); six multiply-adds in place of the Shoup product's
-// ten multiplies, and no conditional subtraction.  With c <= 2^26 a product of |x| <= X 2^60 lies
-// in (-d, 1 + d) 2^60, d = 1.25 (1/4 + X/32).  Forward: [0, 1] grows to (-5.8, 6.8)
-// over four levels.  Inverse: values in (-0.9, 1.9) give sums below 7.6 over two
-// levels, the sums are folded back to [0, 1] there, products stay in (-0.6, 1.6).
-__device__ __forceinline__ void ct_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
-    const uint64_t s = kb_fmul(b, w, c, k28, a);
-    b = (a << 1) - s;
-    a = s;
-}
-
-template <bool RED>
-__device__ __forceinline__ void gs_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
-    const uint64_t u = a + b;
-    b = kb_fmul(a - b, w, c, k28, 0);
-    a = RED ? kb_sfold(u, c) : u;
-}
-
 // ntt_round's options
 enum : int {
     RD_NINV = 1,   // n^-1 multiply at stage 0
@@ -152,7 +132,7 @@ __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, con
 #pragma unroll
         for (int m = 0; m < (1 << j); ++m) {
             const int pos = posc + (kbase + m * (2 * h) * d) * pstep;
-            tws[(1 << j) - 1 + m] = tab[(1 << gst) + (pos >> (log_n - gst))];
+            tws[(1 << j) - 1 + m] = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
         }
     }
 }
@@ -222,7 +202,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     if constexpr (PRE)
                         w = (*pre)[(1 << j) - 1 + m];
                     else
-                        w = tab[(1 << gst) + (pos >> (log_n - gst))];
+                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
 #pragma unroll
                     for (int i = i0; i < i0 + h; ++i) {
                         if constexpr (FOLD)
@@ -250,7 +230,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     if constexpr (PRE)
                         w = (*pre)[(1 << j) - 1 + m];
                     else
-                        w = tab[(1 << gst) + (pos >> (log_n - gst))];
+                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
                     // W1: stage 0 takes the unscaled entry 1, passed in ninv
                     if (W1 && gst == 0) w = ninv;
 #pragma unroll
@@ -810,6 +790,9 @@ uint32_t encode_plan(int col_s, int col_t, int row_t, int col_x, int row_x, int 
            (uint32_t)row_x << 13 | (uint32_t)chunk << 14;
 }
 
+// the word of the built-in plan's shape: the same plan as 0
+uint32_t built_in_word(int log_n) { return encode_plan(col_log_default(log_n), 12, 12, 1, 1); }
+
 int bucket_of(long transforms) {
     return transforms < 64 ? 0 : transforms < 512 ? 1 : transforms < 4096 ? 2 : 3;
 }
@@ -858,15 +841,38 @@ int launch_limb_n(const pass_args &a) {
 // chip is full of tiles either way and the wider rounds' fewer LDS passes win.
 constexpr long SMALL_WORDS = 1L << 19;
 
+// Whether `rows` limbs (more than SMALL_WORDS) take the one-pass kernel.  Its
+// workgroups hold one limb: 8 per CU at 2^12, 4, 2 and 1 at 2^15 (2^16 runs as two
+// halves), so it needs a limb for most CUs, and at 2^15 and 2^16 whole rounds of 256.
+// One pass / two passes, forward, in us:
+//   2^12 165 rows 11.8/15.0, 2040 34.6/57.5       2^13 90 rows 13.7/17.1, 2040 68/115
+//   2^14 60 rows 20.2/16.5, 120 22.6/24.2, 240 27.5/34.2, 2040 159/240
+//   2^15 120 rows 38.9/36.0, 165 40.8/49.7, 255 47.5/68.0, 300 78.1/86.7, 2040 360/501
+//   2^16 165 rows 92.6/83.7, 240 110/113, 255 109/128, 300 198/144, 390 199/187,
+//        510 211/250, 765 340/385, 2040 855/950 (inverse 856/1039)
+bool one_pass(int log_n, long rows) {
+    if (log_n <= 13) return true;
+    if (log_n == 14) return rows >= 112;
+    const long held = 256 * ((rows + 255) / 256);
+    return 100 * rows >= (log_n == 15 ? 57 : 80) * held;
+}
+
 int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, const uint64_t *src, uint64_t *dst,
                   int mod0, int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
                   hipStream_t st, const uint64_t *src2 = nullptr) {
     const plan_fields f = decode_plan(c->log_n, plan);
+    if (plan == built_in_word(c->log_n)) plan = 0;
     const int half = src2 ? batch / 2 : batch;
     if (plan == 0 && ((long)limbs * polys * batch << c->log_n) <= SMALL_WORDS) {
         const pass_args first{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, 0, st, src2, half};
         const pass_args second{c, dst, dst, mod0, limbs, polys, batch, dB, dY, dL, dB, dY, dL, 0, st};
         return small_transform_n(c->log_n, dir, noscale, first, second);
+    }
+    if (plan == 0 && one_pass(c->log_n, (long)limbs * polys * batch)) {
+        bool near60 = true;
+        for (int i = 0; i < limbs; ++i) near60 &= kb_fold_prime(c->mod[mod0 + i]);
+        if (near60)
+            return kb_ntt_reg(c, dir, noscale, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, st, src2, half);
     }
     if (single_pass(c->log_n, f)) {
         const pass_args a{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, f.col_x, st, src2, half};
@@ -1143,27 +1149,27 @@ extern "C" int kbfv_ntt_autotune(kbfv_context *c, int dir, int mod0, int limbs, 
             best_plan = encode_plan(log_n, 0, 0, x, 0);
         }
     }
+    const long N = c->n;
+    auto time_transform = [&](uint32_t plan, float *ms) -> int {
+        auto run = [&]() -> int {
+            return ntt_with_plan(c, dir, false, plan, scratch, scratch, mod0, limbs, polys, 1, 0, (long)limbs * N, N, 0,
+                                 (long)limbs * N, N, st);
+        };
+        KB_TRY(run());
+        KB_HIP(hipEventRecord(e0, st));
+        for (int r = 0; r < reps; ++r) KB_TRY(run());
+        KB_HIP(hipEventRecord(e1, st));
+        KB_HIP(hipEventSynchronize(e1));
+        float t = 0;
+        KB_HIP(hipEventElapsedTime(&t, e0, e1));
+        *ms = t / reps;
+        return KBFV_OK;
+    };
     // chunked two-pass transforms (both passes per chunk of at most 2^(k+23)
     // bytes) with the picked tiles, timed as whole transforms against the
     // unchunked one
     if (rc == KBFV_OK && best_plan != 0 && !single_pass(log_n, decode_plan(log_n, best_plan))) {
-        const long N = c->n;
         const long bytes = (long)polys * limbs * N * 8;
-        auto time_transform = [&](uint32_t plan, float *ms) -> int {
-            auto run = [&]() -> int {
-                return ntt_with_plan(c, dir, false, plan, scratch, scratch, mod0, limbs, polys, 1, 0,
-                                     (long)limbs * N, N, 0, (long)limbs * N, N, st);
-            };
-            KB_TRY(run());
-            KB_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < reps; ++r) KB_TRY(run());
-            KB_HIP(hipEventRecord(e1, st));
-            KB_HIP(hipEventSynchronize(e1));
-            float t = 0;
-            KB_HIP(hipEventElapsedTime(&t, e0, e1));
-            *ms = t / reps;
-            return KBFV_OK;
-        };
         float whole = 0;
         rc = time_transform(best_plan, &whole);
         if (rc == KBFV_OK) best_total = whole;
@@ -1174,6 +1180,12 @@ extern "C" int kbfv_ntt_autotune(kbfv_context *c, int dir, int mod0, int limbs, 
             rc = time_transform(p, &ms);
             if (rc == KBFV_OK && ms < best_total) best_total = ms, best_plan = p;
         }
+    }
+    // the built-in plan, which picks its kernels by size, goes by its shape's word
+    if (rc == KBFV_OK) {
+        float ms = 0;
+        rc = time_transform(0, &ms);
+        if (rc == KBFV_OK && ms < best_total) best_total = ms, best_plan = built_in_word(log_n);
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

@@ -19,7 +19,8 @@ def make(log_n, qn=5):
     d = P.chain60(log_n, qn, 1, 4, 2)
     args = (d["log_n"], d["q"], d["p"], d["t"], d["gamma"], d["plain"])
     tiled = kb.Context(*args)
-    plan = [p for p in kb.ntt_plan_candidates(log_n) if p][0]
+    # tiled passes: two passes, not the built-in plan's word
+    plan = [p for p in kb.ntt_plan_candidates(log_n) if p & 15 != log_n and p >> 12 == 0][0]
     for b in range(kb.lib.kbfv_ntt_plan_bucket(1 << 40) + 1):
         tiled.set_ntt_plan(+1, b, plan)
         tiled.set_ntt_plan(-1, b, plan)

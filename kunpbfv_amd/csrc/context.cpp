@@ -649,7 +649,7 @@ extern "C" int kbfv_context_create(int log_n, const uint64_t *q, int qn, const u
         kbfv_tw *base = tw.data() + (size_t)m * 2 * N;
         for (int i = 0, g = 0; i < N; i++) {
             if (i >= 2 << g) g++;
-            const int k = i < 1 ? 0 : kb_tw_index(log_n, g, i - (1 << g));
+            const int k = i < 1 ? 0 : kb_tw_index(log_n, g, i - (1 << g), kb_fold_prime(qm));
             base[k] = ntt_tw_of(f[i], qm), base[N + k] = ntt_tw_of(iv[i], qm);
         }
         ninv[m] = ntt_tw_of(ni, qm);

@@ -239,11 +239,11 @@ __device__ __forceinline__ void gs_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uin
 }
 
 // Place in a limb's twiddle table of group x of level g (2^g groups): levels follow each
-// other; the last five store the groups of one 32-element block 2^(log_n - 5) apart, so
-// that lanes of consecutive blocks read consecutive twiddles.
-__host__ __device__ __forceinline__ int kb_tw_index(int log_n, int g, int x) {
+// other; of a prime near 2^60 (fold) the last five store the groups of one 32-element block
+// 2^(log_n - 5) apart, so that lanes of consecutive blocks read consecutive twiddles.
+__host__ __device__ __forceinline__ int kb_tw_index(int log_n, int g, int x, bool fold) {
     const int j = g - (log_n - 5);
-    return (1 << g) + (j <= 0 ? x : ((x & ((1 << j) - 1)) << (log_n - 5)) + (x >> j));
+    return (1 << g) + (!fold || j <= 0 ? x : ((x & ((1 << j) - 1)) << (log_n - 5)) + (x >> j));
 }
 // Marks a 32-bit register value as changed.  A multiplicand that a loop reads in
 // every pass is otherwise widened to 64 bits ahead of the loop and takes a

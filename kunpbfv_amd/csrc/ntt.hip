@@ -105,7 +105,7 @@ enum : int {
 // The twiddles of the one butterfly group thread threadIdx.x takes in a round
 // (rounds with exactly one group per thread), in the order the round consumes
 // them: level j of the round, sub-block m -> slot (1 << j) - 1 + m.
-template <int LR, int LOG_S, bool COLUMN, int LOG_T, int VPT = LOG_R>
+template <int LR, int LOG_S, bool COLUMN, int LOG_T, bool FOLD, int VPT = LOG_R>
 __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, const kbfv_tw *tab,
                                                const int log_n, const int g0, const int grp0,
                                                const int stride) {
@@ -132,7 +132,7 @@ __device__ __forceinline__ void round_twiddles(kbfv_tw *tws, const int lam0, con
 #pragma unroll
         for (int m = 0; m < (1 << j); ++m) {
             const int pos = posc + (kbase + m * (2 * h) * d) * pstep;
-            tws[(1 << j) - 1 + m] = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
+            tws[(1 << j) - 1 + m] = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst), FOLD)];
         }
     }
 }
@@ -202,7 +202,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     if constexpr (PRE)
                         w = (*pre)[(1 << j) - 1 + m];
                     else
-                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
+                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst), FOLD)];
 #pragma unroll
                     for (int i = i0; i < i0 + h; ++i) {
                         if constexpr (FOLD)
@@ -230,7 +230,7 @@ __device__ __forceinline__ void ntt_round(uint64_t *tile, const int lam0, const 
                     if constexpr (PRE)
                         w = (*pre)[(1 << j) - 1 + m];
                     else
-                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst))];
+                        w = tab[kb_tw_index(log_n, gst, pos >> (log_n - gst), FOLD)];
                     // W1: stage 0 takes the unscaled entry 1, passed in ninv
                     if (W1 && gst == 0) w = ninv;
 #pragma unroll
@@ -354,7 +354,7 @@ __device__ __forceinline__ void pass_tile(uint64_t *tile, const uint64_t *__rest
             constexpr bool PRE = (C * (S >> LR1) == T);
             if constexpr (PRE) {
                 kbfv_tw pre[(1 << LR1) - 1];
-                round_twiddles<LR1, LOG_S, COLUMN, LOG_T>(pre, LR0, tab, log_n, g0, grp0, stride);
+                round_twiddles<LR1, LOG_S, COLUMN, LOG_T, FOLD>(pre, LR0, tab, log_n, g0, grp0, stride);
                 stage_in<LOG_S, COLUMN, LOG_T>(tile, in, grp0, stride);
                 // pinned here so that the loads are not sunk below the barrier
 #pragma unroll
@@ -406,8 +406,11 @@ __device__ __forceinline__ int xcd_block(int xcd) {
     return (int)blockIdx.x;
 }
 
-// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL
-template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE = false>
+// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL;
+// the launch's moduli are all near 2^60 (FOLD) or none is: one kernel for both, with a
+// branch, holds the registers of the larger (a client's round trip on 35-bit primes,
+// n=16384, 64 messages, 393 us against 378)
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool FOLD>
 __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     k_ntt_pass(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
                const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
@@ -425,15 +428,16 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     const int bi = bid % batch;
     const int l = bid / batch;
     const uint64_t *in = bi < half ? src + bi * sB : src2 + (bi - half) * sB;
-    pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, in + y * sY + l * sL, dst + bi * dB + y * dY + l * dL,
-                                                         tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
+    pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, false, FOLD>(
+        tile, in + y * sY + l * sL, dst + bi * dB + y * dY + l * dL, tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
 }
 
 // A pass for few transforms (the chip is not full and a wave's own chain of
 // butterflies sets the time): four values per thread and tiles of 2^10 (2^11 where
 // a column row would fall below 64 bytes), so a transform spreads over more waves
 // and CUs; radix-4 rounds (and a radix-2 one for an odd count of levels) whose
-// twiddles are all loaded before the data.
+// twiddles are all loaded before the data.  kind0, kind1: bit l for a modulus near 2^60
+// (an argument, so that no load stands before the twiddles' loads).
 // Bound by latency: a launch of 16 K to 240 K words takes 8.3 to 11 us for both
 // passes where the tiles of 2^12 (8 values a thread) take 13 to 16; 8 values with
 // the same preload take 10 to 13.
@@ -445,12 +449,12 @@ struct SmallGeo {
     static constexpr int lr(int k) { return k == NR - 1 && LOG_S % 2 ? 1 : 2; }
 };
 
-template <int LOG_N, int LOG_S, bool COLUMN, bool FWD, bool NOSCALE, int K>
+template <int LOG_N, int LOG_S, bool COLUMN, bool FOLD, int K>
 __device__ __forceinline__ void small_twiddles(kbfv_tw (*pre)[3], const kbfv_tw *tab, int g0, int grp0, int stride) {
     using SG = SmallGeo<LOG_S, COLUMN>;
     if constexpr (K < SG::NR && SG::lr(K) == 2) {
-        round_twiddles<2, LOG_S, COLUMN, SG::LOG_T, SG::VPT>(pre[K], 2 * K, tab, LOG_N, g0, grp0, stride);
-        small_twiddles<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, K + 1>(pre, tab, g0, grp0, stride);
+        round_twiddles<2, LOG_S, COLUMN, SG::LOG_T, FOLD, SG::VPT>(pre[K], 2 * K, tab, LOG_N, g0, grp0, stride);
+        small_twiddles<LOG_N, LOG_S, COLUMN, FOLD, K + 1>(pre, tab, g0, grp0, stride);
     }
 }
 
@@ -484,7 +488,8 @@ __global__ void __launch_bounds__((1 << SmallGeo<LOG_S, COLUMN>::LOG_T) >> 2)
     k_ntt_small(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, const kbfv_tw *__restrict__ tw,
                 const kbfv_tw *__restrict__ ninv_tab, const kbfv_tw *__restrict__ w1_tab,
                 const uint64_t *__restrict__ mods, int mod0, int limbs, int polys, int batch, long sB, long sY,
-                long sL, long dB, long dY, long dL, const uint64_t *__restrict__ src2, int half) {
+                long sL, long dB, long dY, long dL, const uint64_t *__restrict__ src2, int half, uint64_t kind0,
+                uint64_t kind1) {
     using SG = SmallGeo<LOG_S, COLUMN>;
     using G = Geo<LOG_S, COLUMN, SG::LOG_T, SG::VPT>;
     constexpr int groups = (1 << (LOG_N - LOG_S)) / G::C, n = 1 << LOG_N, stride = n >> LOG_S;
@@ -501,16 +506,16 @@ __global__ void __launch_bounds__((1 << SmallGeo<LOG_S, COLUMN>::LOG_T) >> 2)
     const uint64_t *in = (bi < half ? src + bi * sB : src2 + (bi - half) * sB) + y * sY + l * sL;
     uint64_t *out = dst + bi * dB + y * dY + l * dL;
     const kbfv_tw *tab = tw + ((size_t)m * 2 + (FWD ? 0 : 1)) * n;
-    kbfv_tw pre[SG::NR][3];
-    small_twiddles<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, 0>(pre, tab, g0, grp0, stride);
     const uint64_t q = mods[m];
     const kbfv_tw ninv = NI ? ninv_tab[m] : (NOSCALE ? w1_tab[m] : kbfv_tw{0, 0});
-    if constexpr (!FWD && !COLUMN) {
-        stage_in<LOG_S, COLUMN, SG::LOG_T, SG::VPT>(tile, in, grp0, stride);
-        __syncthreads();
-    }
     const auto run = [&](auto fold) {
         constexpr bool FOLD = decltype(fold)::value;
+        kbfv_tw pre[SG::NR][3];
+        small_twiddles<LOG_N, LOG_S, COLUMN, FOLD, 0>(pre, tab, g0, grp0, stride);
+        if constexpr (!FWD && !COLUMN) {
+            stage_in<LOG_S, COLUMN, SG::LOG_T, SG::VPT>(tile, in, grp0, stride);
+            __syncthreads();
+        }
         small_rounds<LOG_N, LOG_S, COLUMN, FWD, NOSCALE, FOLD, 0>(tile, pre, tab, g0, grp0, stride, q, ninv, in, out);
         if constexpr (FWD && !COLUMN) {
 #pragma unroll
@@ -520,7 +525,7 @@ __global__ void __launch_bounds__((1 << SmallGeo<LOG_S, COLUMN>::LOG_T) >> 2)
             }
         }
     };
-    if (kb_fold_prime(q))  // uniform
+    if ((l < 64 ? kind0 : kind1) >> (l & 63) & 1)  // uniform
         run(std::true_type{});
     else
         run(std::false_type{});
@@ -581,13 +586,28 @@ int launch_pass(const pass_args &a) {
         const long groups = (1L << (LOG_N - LOG_S)) / G::C;
         const long blocks = groups * a.limbs * a.polys * a.batch;
         KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
-        hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>), dim3((unsigned)blocks), dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv,
-                           a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB, a.dY,
-                           a.dL, a.xcd, a.src2, a.half);
+        const auto go = [&](auto fold) {
+            constexpr bool FOLD = decltype(fold)::value;
+            hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, FOLD>), dim3((unsigned)blocks),
+                               dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod,
+                               a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd, a.src2,
+                               a.half);
+        };
+        if (kb_fold_prime(a.c->mod[a.mod0]))
+            go(std::true_type{});
+        else
+            go(std::false_type{});
         KB_LAUNCH_CHECK();
         return KBFV_OK;
     }
 }
+
+// Up to this many words a transform under plan 0 takes the small-tile kernels. Both
+// passes together (us, tiles / small tiles): N=2^12 120 rows (480K words) 15.3/12.0,
+// 240 rows 16.9/19.1; N=2^14 30 rows (480K) 15.8/15.0, 60 rows 17.2/23.2; N=2^16 4
+// rows (256K) 16.4/11.7, 8 rows (512K) 15.6/15.0, 15 rows 19.0/22.6. Above it the
+// chip is full of tiles either way and the wider rounds' fewer LDS passes win.
+constexpr long SMALL_WORDS = 1L << 19;
 
 template <int LOG_N, bool COLUMN, bool FWD, bool NOSCALE>
 int launch_small(const pass_args &a) {
@@ -596,9 +616,12 @@ int launch_small(const pass_args &a) {
     using G = Geo<LOG_S, COLUMN, SG::LOG_T, SG::VPT>;
     const long blocks = ((1L << (LOG_N - LOG_S)) / G::C) * a.limbs * a.polys * a.batch;
     KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
+    static_assert(SMALL_WORDS >> 12 <= 128, "one bit per limb in two words");
+    uint64_t kind[2] = {0, 0};
+    for (int l = 0; l < a.limbs; ++l) kind[l >> 6] |= (uint64_t)kb_fold_prime(a.c->mod[a.mod0 + l]) << (l & 63);
     hipLaunchKernelGGL((k_ntt_small<LOG_N, LOG_S, COLUMN, FWD, NOSCALE>), dim3((unsigned)blocks), dim3(G::T), 0, a.st,
                        a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys,
-                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.src2, a.half);
+                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.src2, a.half, kind[0], kind[1]);
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }
@@ -651,7 +674,7 @@ int launch_pass_n(int log_s, int log_t, const pass_args &a) {
     }
 }
 
-// single-pass transform of a whole limb (N <= 2^14: the limb and its row
+// the single-pass plan for primes that k_ntt_reg does not take: a whole limb (N <= 2^14: the limb and its row
 // padding fit in the 160 KB LDS): one HBM read and one write per limb instead
 // of two of each.  Register rounds: radix 16 first, the remaining log N - 4
 // levels in rounds of at most 4 (12: 4,4,4; 13: 4,3,3,3; 14: 4,4,3,3).
@@ -665,17 +688,14 @@ __host__ __device__ constexpr int limb_round_lam(int log_n, int k) {
     return k == 0 ? 0 : limb_round_lam(log_n, k - 1) + limb_round_log(log_n, k - 1);
 }
 
-template <int LOG_N, int K, bool FWD, bool NI, bool FOLD>
+template <int LOG_N, int K, bool FWD, bool NI>
 __device__ __forceinline__ void limb_rounds_mid(uint64_t *tile, const kbfv_tw *tab, uint64_t q, kbfv_tw ninv) {
     // rounds 1 .. limb_rounds - 1, LDS to LDS: ascending (forward) / descending (inverse)
     if constexpr (K >= 1 && K < limb_rounds(LOG_N)) {
         constexpr int KK = FWD ? K : limb_rounds(LOG_N) - K;
-        // the forward transform's last values are folded by the store
-        constexpr int FL = (NI ? RD_NINV : 0) | (FOLD ? RD_FOLD : 0) | (!FWD && K == 1 ? RD_IN : 0) |
-                           (FWD && K == limb_rounds(LOG_N) - 1 ? RD_OPEN : 0);
-        ntt_round<limb_round_log(LOG_N, KK), LOG_N, false, LOG_N, FWD, FL>(tile, limb_round_lam(LOG_N, KK), tab, LOG_N,
-                                                                           0, 0, 1, q, ninv);
-        limb_rounds_mid<LOG_N, K + 1, FWD, NI, FOLD>(tile, tab, q, ninv);
+        ntt_round<limb_round_log(LOG_N, KK), LOG_N, false, LOG_N, FWD, NI ? RD_NINV : 0>(
+            tile, limb_round_lam(LOG_N, KK), tab, LOG_N, 0, 0, 1, q, ninv);
+        limb_rounds_mid<LOG_N, K + 1, FWD, NI>(tile, tab, q, ninv);
     }
 }
 
@@ -702,31 +722,22 @@ __global__ void __launch_bounds__((1 << LOG_N) >> LOG_R)
     uint64_t *out = dst + bi * dB + y * dY + l * dL;
     constexpr bool NI = !FWD && !NOSCALE;
     const kbfv_tw ninv = NI ? ninv_tab[m] : (NOSCALE ? w1_tab[m] : kbfv_tw{0, 0});
-    const auto run = [&](auto fold) {
-        constexpr bool FOLD = decltype(fold)::value;
-        constexpr int FD = FOLD ? RD_FOLD : 0;
-        if constexpr (FWD) {
-            // the radix-16 round of stride N/16 reads global memory in 128-byte runs
-            ntt_round<4, LOG_N, false, LOG_N, true, FD | RD_GIN | RD_IN>(tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, in);
-            limb_rounds_mid<LOG_N, 1, true, false, FOLD>(tile, tab, q, ninv);
+    if constexpr (FWD) {
+        // the radix-16 round of stride N/16 reads global memory in 128-byte runs
+        ntt_round<4, LOG_N, false, LOG_N, true, RD_GIN>(tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, in);
+        limb_rounds_mid<LOG_N, 1, true, false>(tile, tab, q, ninv);
 #pragma unroll
-            for (int j = 0; j < n / T; ++j) {
-                const int k = threadIdx.x + j * T;
-                out[k] = forward_canon<FOLD>(tile[G::addr(0, k)], q);
-            }
-        } else {
-            stage_in<LOG_N, false, LOG_N>(tile, in, 0, 1);
-            __syncthreads();
-            limb_rounds_mid<LOG_N, 1, false, NI, FOLD>(tile, tab, q, ninv);
-            ntt_round<4, LOG_N, false, LOG_N, false,
-                      FD | (NI ? RD_NINV : 0) | RD_GOUT | (NOSCALE ? RD_W1 : RD_FIN)>(tile, 0, tab, LOG_N, 0, 0, 1, q,
-                                                                                     ninv, nullptr, out);
+        for (int j = 0; j < n / T; ++j) {
+            const int k = threadIdx.x + j * T;
+            out[k] = forward_canon<false>(tile[G::addr(0, k)], q);
         }
-    };
-    if (kb_fold_prime(q))  // uniform
-        run(std::true_type{});
-    else
-        run(std::false_type{});
+    } else {
+        stage_in<LOG_N, false, LOG_N>(tile, in, 0, 1);
+        __syncthreads();
+        limb_rounds_mid<LOG_N, 1, false, NI>(tile, tab, q, ninv);
+        ntt_round<4, LOG_N, false, LOG_N, false, (NI ? RD_NINV : 0) | RD_GOUT | (NOSCALE ? RD_W1 : RD_FIN)>(
+            tile, 0, tab, LOG_N, 0, 0, 1, q, ninv, nullptr, out);
+    }
 }
 
 // forward column pass of the external product's digit polynomials, the digit
@@ -834,13 +845,6 @@ int launch_limb_n(const pass_args &a) {
     }
 }
 
-// Up to this many words a transform under plan 0 takes the small-tile kernels. Both
-// passes together (us, tiles / small tiles): N=2^12 120 rows (480K words) 15.3/12.0,
-// 240 rows 16.9/19.1; N=2^14 30 rows (480K) 15.8/15.0, 60 rows 17.2/23.2; N=2^16 4
-// rows (256K) 16.4/11.7, 8 rows (512K) 15.6/15.0, 15 rows 19.0/22.6. Above it the
-// chip is full of tiles either way and the wider rounds' fewer LDS passes win.
-constexpr long SMALL_WORDS = 1L << 19;
-
 // Whether `rows` limbs (more than SMALL_WORDS) take the one-pass kernel.  Its
 // workgroups hold one limb: 8 per CU at 2^12, 4, 2 and 1 at 2^15 (2^16 runs as two
 // halves), so it needs a limb for most CUs, and at 2^15 and 2^16 whole rounds of 256.
@@ -868,12 +872,17 @@ int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, c
         const pass_args second{c, dst, dst, mod0, limbs, polys, batch, dB, dY, dL, dB, dY, dL, 0, st};
         return small_transform_n(c->log_n, dir, noscale, first, second);
     }
-    if (plan == 0 && one_pass(c->log_n, (long)limbs * polys * batch)) {
-        bool near60 = true;
-        for (int i = 0; i < limbs; ++i) near60 &= kb_fold_prime(c->mod[mod0 + i]);
-        if (near60)
-            return kb_ntt_reg(c, dir, noscale, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, st, src2, half);
+    // one kind of prime per launch below
+    const bool near60 = kb_fold_prime(c->mod[mod0]);
+    int run = 1;
+    while (run < limbs && kb_fold_prime(c->mod[mod0 + run]) == near60) ++run;
+    if (run < limbs) {
+        KB_TRY(ntt_with_plan(c, dir, noscale, plan, src, dst, mod0, run, polys, batch, sB, sY, sL, dB, dY, dL, st, src2));
+        return ntt_with_plan(c, dir, noscale, plan, src + run * sL, dst + run * dL, mod0 + run, limbs - run, polys, batch,
+                             sB, sY, sL, dB, dY, dL, st, src2 ? src2 + run * sL : nullptr);
     }
+    if (near60 && (plan == 0 ? one_pass(c->log_n, (long)limbs * polys * batch) : single_pass(c->log_n, f)))
+        return kb_ntt_reg(c, dir, noscale, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, st, src2, half);
     if (single_pass(c->log_n, f)) {
         const pass_args a{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, f.col_x, st, src2, half};
         if (dir > 0) return launch_limb_n<true, false>(a);
@@ -1130,25 +1139,6 @@ extern "C" int kbfv_ntt_autotune(kbfv_context *c, int dir, int mod0, int limbs, 
             best_plan = encode_plan(cs, bct, brt, bcx, brx);
         }
     }
-    // one launch per transform where the limb fits a workgroup's LDS
-    for (int x = 0; x <= 1 && rc == KBFV_OK && log_n <= 14; ++x) {
-        const long N = c->n;
-        const pass_args a{c, scratch, scratch, mod0, limbs, polys, 1, 0, (long)limbs * N, N, 0, (long)limbs * N, N, x,
-                          st};
-        auto run = [&]() -> int { return dir > 0 ? launch_limb_n<true, false>(a) : launch_limb_n<false, false>(a); };
-        rc = run();
-        if (rc == KBFV_OK) rc = hipEventRecord(e0, st) == hipSuccess ? KBFV_OK : KBFV_EHIP;
-        for (int r = 0; r < reps && rc == KBFV_OK; ++r) rc = run();
-        if (rc == KBFV_OK) rc = hipEventRecord(e1, st) == hipSuccess ? KBFV_OK : KBFV_EHIP;
-        if (rc == KBFV_OK) rc = hipEventSynchronize(e1) == hipSuccess ? KBFV_OK : KBFV_EHIP;
-        float t = 0;
-        if (rc == KBFV_OK) rc = hipEventElapsedTime(&t, e0, e1) == hipSuccess ? KBFV_OK : KBFV_EHIP;
-        if (rc == KBFV_EHIP) kb_set_error("NTT autotune: HIP event call failed");
-        if (rc == KBFV_OK && t / reps < best_total) {
-            best_total = t / reps;
-            best_plan = encode_plan(log_n, 0, 0, x, 0);
-        }
-    }
     const long N = c->n;
     auto time_transform = [&](uint32_t plan, float *ms) -> int {
         auto run = [&]() -> int {
@@ -1165,6 +1155,12 @@ extern "C" int kbfv_ntt_autotune(kbfv_context *c, int dir, int mod0, int limbs, 
         *ms = t / reps;
         return KBFV_OK;
     };
+    // one launch per transform where the limb fits a workgroup
+    for (int x = 0; x <= 1 && rc == KBFV_OK && log_n <= 14; ++x) {
+        float ms = 0;
+        rc = time_transform(encode_plan(log_n, 0, 0, x, 0), &ms);
+        if (rc == KBFV_OK && ms < best_total) best_total = ms, best_plan = encode_plan(log_n, 0, 0, x, 0);
+    }
     // chunked two-pass transforms (both passes per chunk of at most 2^(k+23)
     // bytes) with the picked tiles, timed as whole transforms against the
     // unchunked one

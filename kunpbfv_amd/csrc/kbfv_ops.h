@@ -70,6 +70,8 @@ kb_stream_key kb_stream_setup(const uint8_t seed[32], uint64_t tag);
 // kind: 0 uniform, 1 ternary, 2 zero-one, 3 CBD.  out [batch][limbs][N]; batch entry b reads
 // stream entry entry0 + b (XSalsa20 nonce bytes 16..23).
 // ostride: elements between batch entries (<= 0: limbs*N, contiguous)
+int kb_enc_sample(const kbfv_context *c, const uint8_t seed[32], uint64_t tag_v, uint64_t tag_e0, uint64_t tag_e1,
+                  const uint64_t *m, uint64_t *out, int batch, hipStream_t st);
 int kb_sample(const kbfv_context *c, int kind, const uint8_t seed[32], uint64_t tag, uint64_t entry0,
               int mod0, int limbs, uint64_t *out, long ostride, int batch, hipStream_t st);
 int kb_xsalsa20(const uint8_t key[32], const uint8_t nonce[24], uint64_t block0, uint8_t *out, size_t len,

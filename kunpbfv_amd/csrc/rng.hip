@@ -130,6 +130,68 @@ __global__ void k_sample(kb_dev_tables t, kb_stream_key key, uint64_t entry0,
     }
 }
 
+// Encryption's three noise polynomials over Q in one launch: v (zero-one), e0 (CBD) and
+// e1 + Delta m (Delta m = [-Q m]_t t^-1, as in k_delta_m).  The samples are those
+// of k_sample's streams.  A workgroup draws 512 coefficients, one Salsa20 block per
+// thread (8 for v, 64 for e0, 64 for e1), keeps them in LDS as bytes and writes them to
+// every limb in 16-byte words, where a thread per block wrote its 8 or 64 neighbours
+// with a stride between lanes: 24 messages of 6 limbs, n=16384, 64 + 2 x 22 us and 29
+// for Delta m and its sum against 21.  grid (n / 512, batch)
+constexpr int ENC_RUN = 512;
+typedef uint64_t word2 __attribute__((ext_vector_type(2), aligned(8)));  // scratch need not be 16-byte aligned
+__global__ void __launch_bounds__(192)
+    k_enc_sample(kb_dev_tables t, kb_stream_key kv, kb_stream_key k0, kb_stream_key k1, const uint64_t *__restrict__ m,
+                 uint64_t *__restrict__ out, uint64_t plain, uint64_t negq, uint64_t negq_s, int qn, int oQ, int n,
+                 long poly) {
+    __shared__ int8_t smp[3][ENC_RUN];
+    __shared__ uint64_t mq[ENC_RUN];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int bt = blockIdx.y, run = blockIdx.x;
+    // wave 0: v, 1: e0, 2: e1
+    if (wave != 0 || lane < 8) {
+        kb_stream_key key = wave == 0 ? kv : wave == 1 ? k0 : k1;
+        key.n8[0] = (uint32_t)bt;
+        key.n8[1] = 0;
+        uint32_t z[16];
+        salsa_block(key, (uint64_t)run * (wave == 0 ? 8 : 64) + lane, z);
+        if (wave == 0) {
+#pragma unroll
+            for (int s = 0; s < 64; ++s) {
+                const uint32_t byte = (z[s >> 2] >> (8 * (s & 3))) & 0xffu;
+                smp[0][lane * 64 + s] = byte < 128 ? 0 : (byte < 192 ? 1 : -1);
+            }
+        } else {
+            const uint64_t M = (1ULL << 21) - 1;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const uint64_t x = w64(z, s);
+                smp[wave][lane * 8 + s] = (int8_t)(__popcll(x & M) - __popcll((x >> 21) & M));
+            }
+        }
+    }
+    const long k0c = (long)run * ENC_RUN;
+    for (int i = threadIdx.x; i < ENC_RUN; i += 192) mq[i] = kb_shoup(m[(long)bt * n + k0c + i], negq, negq_s, plain);
+    __syncthreads();
+    for (int w = wave; w < 3 * qn; w += 3) {  // one limb of one polynomial per wave
+        const int which = w / qn, l = w - which * qn;
+        const uint64_t q = t.mod[oQ + l];
+        const kbfv_tw ti = t.tinv_mod_q[l];
+        uint64_t *o = out + which * poly + ((long)bt * qn + l) * n + k0c;
+#pragma unroll
+        for (int i = 0; i < ENC_RUN / 128; ++i) {
+            const int k = i * 128 + lane * 2;
+            word2 v;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int x = smp[which][k + j];
+                v[j] = x < 0 ? q - (uint64_t)(-x) : (uint64_t)x;
+                if (which == 2) v[j] = kb_addmod(v[j], kb_shoup(mq[k + j], ti.w, ti.ws, q), q);
+            }
+            *(word2 *)(o + k) = v;
+        }
+    }
+}
+
 }  // namespace
 
 kb_stream_key kb_stream_setup(const uint8_t seed[32], uint64_t tag) {
@@ -197,6 +259,18 @@ int kb_sample(const kbfv_context *c, int kind, const uint8_t seed[32], uint64_t 
         case 2: hipLaunchKernelGGL(k_sample<2>, grid, dim3(256), 0, st, c->t, key, entry0, out, ostride, mod0, limbs, c->n, per); break;
         default: hipLaunchKernelGGL(k_sample<3>, grid, dim3(256), 0, st, c->t, key, entry0, out, ostride, mod0, limbs, c->n, per); break;
     }
+    KB_LAUNCH_CHECK();
+    return KBFV_OK;
+}
+
+// out: v | e0 | e1 + Delta m, each [batch][qn][N]
+int kb_enc_sample(const kbfv_context *c, const uint8_t seed[32], uint64_t tag_v, uint64_t tag_e0, uint64_t tag_e1,
+                  const uint64_t *m, uint64_t *out, int batch, hipStream_t st) {
+    KB_REQUIRE(c && seed && m && out && batch > 0 && batch <= 65535, "bad sampler arguments");
+    static_assert((1 << 12) % ENC_RUN == 0, "whole runs at every ring degree");
+    hipLaunchKernelGGL(k_enc_sample, dim3(c->n / ENC_RUN, batch), dim3(192), 0, st, c->t, kb_stream_setup(seed, tag_v),
+                       kb_stream_setup(seed, tag_e0), kb_stream_setup(seed, tag_e1), m, out, c->plain, c->negQ_mod_t,
+                       c->negQ_mod_t_shoup, c->qn, c->oQ, c->n, (long)batch * c->qn * c->n);
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }

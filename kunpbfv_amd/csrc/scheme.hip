@@ -451,35 +451,22 @@ extern "C" int kbfv_keygen_swk(const kbfv_context *c, const uint8_t seed[32], co
 }
 
 // ---------------------------------------------------------------- encrypt / decrypt
-static size_t enc_layout(const kbfv_context *c, int batch, void *base, uint64_t **v, uint64_t **e0,
-                         uint64_t **u1, uint64_t **dm) {
-    const size_t L = (size_t)c->qn * c->n * batch;
-    Bump bp(base);
-    uint64_t *p0 = bp.take(L), *p1 = bp.take(L), *p2 = bp.take(L), *p3 = bp.take(L);
-    if (v) *v = p0, *e0 = p1, *u1 = p2, *dm = p3;
-    return bp.used;
-}
+// v | e0 | e1 + Delta m of a batch, and as much again as one of them that callers have
+// sized their scratch for
 extern "C" size_t kbfv_encrypt_workspace_bytes(const kbfv_context *c, int batch) {
-    return (c && batch > 0) ? enc_layout(c, batch, nullptr, nullptr, nullptr, nullptr, nullptr) : 0;
+    return (c && batch > 0) ? 4 * sizeof(uint64_t) * (size_t)c->qn * c->n * batch : 0;
 }
 
 extern "C" int kbfv_encrypt(const kbfv_context *c, const uint8_t seed[32], const uint64_t *pk, const uint64_t *m,
                             uint64_t *ct, int batch, void *ws, size_t ws_bytes, void *st) {
     KB_REQUIRE(c && seed && pk && m && ct && ws && batch > 0, "null argument");
     KB_REQUIRE(ws_bytes >= kbfv_encrypt_workspace_bytes(c, batch), "workspace too small");
-    uint64_t *v, *e0, *u1, *dm;
-    enc_layout(c, batch, ws, &v, &e0, &u1, &dm);
     const int qn = c->qn;
-    hipStream_t s = S(st);
-    KB_TRY(kb_sample(c, 2, seed, TAG(TAG_ENC_V), 0, c->oQ, qn, v, 0, batch, s));
-    KB_TRY(kb_sample(c, 3, seed, TAG(TAG_ENC_E0), 0, c->oQ, qn, e0, 0, batch, s));
-    KB_TRY(kb_sample(c, 3, seed, TAG(TAG_ENC_E1), 0, c->oQ, qn, u1, 0, batch, s));
-    KB_TRY(kb_delta_m(c, m, dm, batch, s));
-    KB_TRY(kb_poly_binop(c, 0, u1, dm, u1, c->oQ, qn, batch, s));  // e1 + Delta*m
-    KB_TRY(kb_ntt_inplace(c, +1, v, c->oQ, qn, batch, s));
-    KB_TRY(kb_ntt_inplace(c, +1, e0, c->oQ, qn, batch, s));
-    KB_TRY(kb_ntt_inplace(c, +1, u1, c->oQ, qn, batch, s));
     const long total = (long)batch * qn * c->n;
+    uint64_t *v = (uint64_t *)ws, *e0 = v + total, *u1 = e0 + total;
+    hipStream_t s = S(st);
+    KB_TRY(kb_enc_sample(c, seed, TAG(TAG_ENC_V), TAG(TAG_ENC_E0), TAG(TAG_ENC_E1), m, v, batch, s));
+    KB_TRY(kb_ntt_inplace(c, +1, v, c->oQ, qn, 3 * batch, s));
     hipLaunchKernelGGL(k_enc_combine, dim3(blocks_for(total, BS)), dim3(BS), 0, s, c->t, v, e0, u1, pk, ct, qn,
                        c->oQ, c->n, total);
     KB_LAUNCH_CHECK();

@@ -179,7 +179,7 @@ __device__ __forceinline__ void kb_mad(int64_t &acc, int a, int b) {
     acc = (int64_t)((uint64_t)acc + (uint64_t)((int64_t)a * b));
 }
 __device__ __forceinline__ void kb_mad(uint64_t &acc, uint32_t a, uint32_t b) { acc += (uint64_t)a * b; }
-// Multiplication modulo a prime q = 2^60 - c, 0 < c <= 2^26, on signed values.  x =
+// Multiplication modulo a prime q = 2^60 - c, 0 < c < 2^28, on signed values.  x =
 // x1 2^32 + x0 with x0 signed; the constant w (twiddle) and w' = w 2^32 mod q are
 // split at 28 bits into signed 32-bit halves, w = w1 2^28 + w0.  Then
 // x w = x0 w + x1 w' = A + 2^28 B, A = x0 w0 + x1 w'0, B = x0 w1 + x1 w'1, and with
@@ -187,7 +187,7 @@ __device__ __forceinline__ void kb_mad(uint64_t &acc, uint32_t a, uint32_t b) { 
 // Six multiply-adds with no carry between them.  |w|, |w'| <= 2^59 and |w0|, |w'0| <=
 // 2^27, so for |x| < 8 (2^60 - 2^32) B stays below 2^63 and for |x| <= X 2^60 the result
 // lies between -d 2^60 and (1 + d) 2^60, d = (1/4 + X/32) (1 + c 2^-28).
-__host__ __device__ __forceinline__ bool kb_fold_prime(uint64_t q) { return (q >> 26) == (1ULL << 34) - 1; }
+__host__ __device__ __forceinline__ bool kb_fold_prime(uint64_t q) { return (q >> 28) == (1ULL << 32) - 1; }
 __device__ __forceinline__ uint32_t kb_fold_c(uint64_t q) { return (uint32_t)((1ULL << 60) - q); }
 // x w + add, w as a pair of packed halves (w0 | w1 << 32); k28 = 2^28
 __device__ __forceinline__ uint64_t kb_fmul(uint64_t x, kbfv_tw w, uint32_t c, uint32_t k28, uint64_t add) {
@@ -218,13 +218,14 @@ __device__ __forceinline__ uint64_t kb_ufold(uint64_t x, uint32_t c) {
 __device__ __forceinline__ uint64_t kb_fold_canon(uint64_t x, uint64_t q, uint64_t nq, uint32_t c) {
     return kb_csub_sel(kb_ufold(x + (q << 3), c), nq);
 }
-// Butterflies for primes 2^60 - c, c < 2^26: values are signed, twiddles signed
+// Butterflies for primes 2^60 - c, c < 2^28: values are signed, twiddles signed
 // halves (kb_fmul).  The product comes on top of its addend, so the sum is free and
 // the difference is 2a - (a + t); six multiply-adds in place of the Shoup product's
-// ten multiplies, and no conditional subtraction.  With c <= 2^26 a product of |x| <= X 2^60 lies
-// in (-d, 1 + d) 2^60, d = 1.25 (1/4 + X/32).  Forward: [0, 1] grows to (-5.8, 6.8)
-// over four levels.  Inverse: values in (-0.9, 1.9) give sums below 7.6 over two
-// levels, the sums are folded back to [0, 1] there, products stay in (-0.6, 1.6).
+// ten multiplies, and no conditional subtraction.  A product of |x| <= X 2^60 lies in
+// (-d, 1 + d) 2^60, d < 1/2 + X/16.  Forward: [0, 1] grows over four levels to (-1.6,
+// 2.6), (-3.3, 4.3), (-5.0, 6.0), (-6.9, 7.9).  Inverse: values in (-0.9, 1.9) give sums
+// below 7.6 over two levels, the sums are folded back to [0, 1] there, the products of
+// differences below 5.7 stay in (-0.9, 1.9).
 __device__ __forceinline__ void ct_fold(uint64_t &a, uint64_t &b, kbfv_tw w, uint32_t c, uint32_t k28) {
     const uint64_t s = kb_fmul(b, w, c, k28, a);
     b = (a << 1) - s;

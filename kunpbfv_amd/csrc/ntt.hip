@@ -13,7 +13,7 @@
 //                   global stages 0 .. log2(N1)-1
 //   row pass     -- C contiguous chunks of N2 elements, remaining stages
 // Forward = column then row; inverse = row then column.  Butterflies modulo primes
-// 2^60 - c (c <= 2^26, the chains of 60-bit primes) work on signed values with ten
+// 2^60 - c (c < 2^28, the chains of 60-bit primes) work on signed values with ten
 // instructions and no conditional subtraction; a register round folds its values
 // back to 60 bits.  Modulo other primes values stay lazy in
 // [0, 8q) (forward) / [0, 4q) (inverse) between stages (moduli are below 2^60,

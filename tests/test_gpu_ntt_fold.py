@@ -1,4 +1,4 @@
-"""GPU: transforms modulo primes 2^60 - c run on signed values for c up to 2^26 and on
+"""GPU: transforms modulo primes 2^60 - c run on signed values for c up to 2^28 and on
 Shoup products past it: primes on both sides of that line and a large one in one
 launch, every ring degree, residues at the ends of their range, against the oracle;
 the unscaled inverse and long sums inside HomMult are covered by its own tests."""
@@ -14,9 +14,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("log_n", [12, 13, 14, 15, 16])
 def test_both_sides_of_the_line(log_n):
     import kunpbfv_amd as kb
-    m, line = 1 << 17, (1 << 60) - (1 << 26)
-    below = orc.primes_descending(line, m, 2)  # c just above 2^26
-    above = orc.primes_descending(line + 64 * m, m, 64)  # c just below 2^26
+    m, line = 1 << 17, (1 << 60) - (1 << 28)
+    below = orc.primes_descending(line, m, 2)  # c just above 2^28
+    above = orc.primes_descending(line + 512 * m, m, 64)  # c just below 2^28
     above = sorted(v for v in above if v > line)[:2]
     assert len(above) == 2
     q = [above[0], below[0], orc.primes_descending(1 << 60, m, 8)[7], above[1], below[1]]

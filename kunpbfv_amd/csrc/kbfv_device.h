@@ -214,6 +214,16 @@ __device__ __forceinline__ uint64_t kb_ufold(uint64_t x, uint32_t c) {
     const uint32_t hi = (uint32_t)(x >> 32);
     return kb_mad32(hi >> 28, c, ((uint64_t)(hi & 0x0fffffffu) << 32) | (uint32_t)x);
 }
+// v below 2^122 modulo a prime 2^60 - c, c < 2^28: v = H 2^60 + L is H c + L; of H c's
+// upper word product u 2^28 + w the part u 2^60 folds once more.  Half the multiplies of
+// a Barrett reduction.
+__device__ __forceinline__ uint64_t kb_fold128(kbfv_u128 v, uint32_t c, uint64_t nq) {
+    const uint64_t H = v.hi << 4 | v.lo >> 60, L = v.lo & ((1ULL << 60) - 1);
+    const uint64_t p = (uint64_t)(uint32_t)(H >> 32) * c;
+    const uint64_t w = (uint64_t)((uint32_t)p & 0x0fffffffu) << 32;
+    const uint64_t r = kb_mad32((uint32_t)(p >> 28), c, kb_mad32((uint32_t)H, c, L) + w);  // < 2^62
+    return kb_csub_sel(kb_ufold(r, c), nq);
+}
 // signed x, |x| <= 7.9 2^60 -> [0, q)
 __device__ __forceinline__ uint64_t kb_fold_canon(uint64_t x, uint64_t q, uint64_t nq, uint32_t c) {
     return kb_csub_sel(kb_ufold(x + (q << 3), c), nq);

@@ -44,7 +44,7 @@ int kb_inner_product_mfma(const kbfv_context *c, const uint64_t *cin, const uint
                           int batch, hipStream_t st);
 int kb_modup_t_to_pq(const kbfv_context *c, const uint64_t *in, uint64_t *out, int batch, hipStream_t st);
 int kb_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, const uint64_t *add,
-               long add_stride, int batch, hipStream_t st);
+               long add_stride, int batch, hipStream_t st, int add_h = 0);
 // kb_modup_t_to_pq then kb_moddown in one kernel, without the PQ intermediate,
 // for the shapes kb_modup_moddown_fused accepts; other shapes run the two
 // kernels through pq_tmp ([batch][2][pn+qn][N], unused and may be null when fused)
@@ -55,8 +55,9 @@ int kb_modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, c
 // (NTT over T, left as it is) -> INTT over T into ip_coeff (same shape) ->
 // modUp T->PQ and modDown into out [batch][2][qn][N] (+ add).  For the fused
 // shapes the INTT leaves out n^-1 and the modUp folds it into its constants.
+// add joins the polynomials from add_h on (0: both, 1: the second).
 int kb_ks_tail(const kbfv_context *c, const uint64_t *ip, uint64_t *ip_coeff, uint64_t *out, const uint64_t *add,
-               long add_stride, int batch, uint64_t *pq_tmp, hipStream_t st);
+               long add_stride, int batch, uint64_t *pq_tmp, hipStream_t st, int add_h = 0);
 // digit decomposition of the Q limbs into T followed by the forward NTT over T
 int kb_digits_to_t_ntt(const kbfv_context *c, const uint64_t *x_coeff, long x_stride, uint64_t *out,
                        int batch, uint64_t *tmp, hipStream_t st);

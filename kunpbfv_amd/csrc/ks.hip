@@ -122,7 +122,7 @@ __global__ void k_modup_t_to_pq(kb_dev_tables t, const uint64_t *__restrict__ in
 // in [batch][2][pq][N] -> out [batch][2][qn][N] (+ add [batch](2 polys at add_stride))
 // grid (n / KS_BS, qn, batch * 2): coefficient, limb l, ciphertext-poly (bt*2 + h)
 __global__ void k_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
-                          const uint64_t *__restrict__ add, long add_stride, int pn, int qn, int oQ,
+                          const uint64_t *__restrict__ add, long add_stride, int add_h, int pn, int qn, int oQ,
                           int n) {
     const int k = blockIdx.x * KS_BS + threadIdx.x;
     const int l = blockIdx.y;
@@ -148,7 +148,7 @@ __global__ void k_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint
     ra = q - ra + ip[(long)(pn + l) * n];
     const kbfv_tw pi = t.Pinv_mod_q[l];
     uint64_t v = kb_shoup(ra, pi.w, pi.ws, q);
-    if (add) v = kb_addmod(v, add[bt * add_stride + ((long)h * qn + l) * n + k], q);
+    if (add && h >= add_h) v = kb_addmod(v, add[bt * add_stride + ((long)h * qn + l) * n + k], q);
     out[(rest * qn + l) * (long)n + k] = v;
 }
 
@@ -158,7 +158,8 @@ __global__ void k_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint
 // ri blocks in index order, P limbs first, so the thread keeps the PN special
 // residues in registers and finishes each Q limb's modDown as soon as its
 // modUp value exists: the [2][pn+qn] PQ polynomials never reach memory.  The
-// arithmetic of every limb is that of k_modup_t_to_pq then k_moddown.  TN, G
+// arithmetic of every limb is that of k_modup_t_to_pq then k_moddown, its 128-bit sums
+// folded at bit 60 where the limb's prime is near 2^60.  TN, G
 // and PN (tn, gamma, pn) are compile-time so that the per-thread arrays stay
 // in registers.  NOSC: the input is N times the INTT (lazy, below 4t); the
 // first step [(x + T/2) (T/t)^-1]_t is a Shoup product exact for any 64-bit
@@ -166,8 +167,8 @@ __global__ void k_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint
 // same canonical value.  grid (n / KS_BS, batch * 2)
 template <int TN, int G, int PN, bool NOSC>
 __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
-                                const uint64_t *__restrict__ add, long add_stride, int qn, int B, int oQ,
-                                int oT, int n) {
+                                const uint64_t *__restrict__ add, long add_stride, int add_h, int qn, int B,
+                                int oQ, int oT, int n) {
     const int k = blockIdx.x * KS_BS + threadIdx.x;
     const long rest = blockIdx.y;
     const int h = (int)(rest & 1);
@@ -208,7 +209,8 @@ __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in
 #pragma unroll
             for (int kk = 0; kk < TN; ++kk) kb_mac128(acc, rb[kk], t.t_hat_mod_pq[idx * TN + kk]);
             kb_sub128(acc, (uint64_t)vf * t.t_mod_pq[idx]);
-            uint64_t v = kb_barrett128(acc, r, t.mu[2 * idx], t.mu[2 * idx + 1]);
+            uint64_t v = kb_fold_prime(r) ? kb_fold128(acc, kb_fold_c(r), 0 - r)
+                                          : kb_barrett128(acc, r, t.mu[2 * idx], t.mu[2 * idx + 1]);
             v = kb_csub(v + r - t.halfT_mod[idx], r);
             if (idx < PN) {
 #pragma unroll
@@ -222,7 +224,8 @@ __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in
             const uint64_t q = t.mod[m], mlo = t.mu[2 * m], mhi = t.mu[2 * m + 1];
             uint64_t ra;
             if constexpr (PN == 1) {
-                ra = kb_barrett128(kbfv_u128{xp[0], 0}, q, mlo, mhi);
+                // below 2^60: less than 2q where q is near 2^60
+                ra = kb_fold_prime(q) ? kb_csub_sel(xp[0], 0 - q) : kb_barrett128(kbfv_u128{xp[0], 0}, q, mlo, mhi);
             } else {
                 kbfv_u128 a2{0, 0};
 #pragma unroll
@@ -231,12 +234,12 @@ __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in
                     const uint64_t rp = kb_shoup(xp[jj], hi.w, hi.ws, t.mod[jj]);
                     kb_mac128(a2, rp, t.p_hat_mod_q[l * PN + jj]);
                 }
-                ra = kb_barrett128(a2, q, mlo, mhi);
+                ra = kb_fold_prime(q) ? kb_fold128(a2, kb_fold_c(q), 0 - q) : kb_barrett128(a2, q, mlo, mhi);
             }
             ra = q - ra + v;
             const kbfv_tw pi = t.Pinv_mod_q[l];
             uint64_t o = kb_shoup(ra, pi.w, pi.ws, q);
-            if (add) o = kb_addmod(o, add[bt * add_stride + ((long)h * qn + l) * n + k], q);
+            if (add && h >= add_h) o = kb_addmod(o, add[bt * add_stride + ((long)h * qn + l) * n + k], q);
             out[(rest * qn + l) * (long)n + k] = o;
         }
     }
@@ -251,14 +254,15 @@ bool kb_modup_moddown_fused(const kbfv_context *c) {
 }
 
 static int modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, const uint64_t *add,
-                         long add_stride, int batch, uint64_t *pq_tmp, bool nosc, hipStream_t st) {
+                         long add_stride, int add_h, int batch, uint64_t *pq_tmp, bool nosc, hipStream_t st) {
     KB_REQUIRE(c && in && out && batch > 0, "bad modUp/modDown arguments");
     KB_REQUIRE(2L * batch <= 65535, "batch too large for one modUp/modDown launch");
     // PN special residues first: the P limbs must all lie before any Q limb
 #define KB_MUMD(TN_, G_, PN_, NOSC_)                                                                       \
     if (c->tn == TN_ && c->gamma == G_ && c->pn == PN_ && nosc == NOSC_) {                                 \
         hipLaunchKernelGGL((k_modup_moddown<TN_, G_, PN_, NOSC_>), dim3(c->n / KS_BS, 2 * batch), dim3(KS_BS), \
-                           0, st, c->t, in, out, add, add_stride, c->qn, c->ri_blocks, c->oQ, c->oT, c->n); \
+                           0, st, c->t, in, out, add, add_stride, add_h, c->qn, c->ri_blocks, c->oQ, c->oT,  \
+                           c->n);                                                                            \
         KB_LAUNCH_CHECK();                                                                                 \
         return KBFV_OK;                                                                                    \
     }
@@ -276,16 +280,16 @@ static int modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *ou
     KB_REQUIRE(pq_tmp, "modUp/modDown of this shape needs a PQ buffer");
     const int rc = kb_modup_t_to_pq(c, in, pq_tmp, batch, st);
     if (rc != KBFV_OK) return rc;
-    return kb_moddown(c, pq_tmp, out, add, add_stride, batch, st);
+    return kb_moddown(c, pq_tmp, out, add, add_stride, batch, st, add_h);
 }
 
 int kb_modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, const uint64_t *add,
                      long add_stride, int batch, uint64_t *pq_tmp, hipStream_t st) {
-    return modup_moddown(c, in, out, add, add_stride, batch, pq_tmp, false, st);
+    return modup_moddown(c, in, out, add, add_stride, 0, batch, pq_tmp, false, st);
 }
 
 int kb_ks_tail(const kbfv_context *c, const uint64_t *ip, uint64_t *ip_coeff, uint64_t *out, const uint64_t *add,
-               long add_stride, int batch, uint64_t *pq_tmp, hipStream_t st) {
+               long add_stride, int batch, uint64_t *pq_tmp, hipStream_t st, int add_h) {
     KB_REQUIRE(c && ip && ip_coeff && out && batch > 0, "bad key-switch arguments");
     const long N = c->n, TS = (long)c->tn * N;
     const int polys = 2 * c->ri_blocks * batch;
@@ -293,7 +297,7 @@ int kb_ks_tail(const kbfv_context *c, const uint64_t *ip, uint64_t *ip_coeff, ui
     const int rc = nosc ? kb_intt_noscale(c, ip, ip_coeff, c->oT, c->tn, polys, 1, 0, TS, N, 0, TS, N, st)
                         : kb_ntt(c, -1, ip, ip_coeff, c->oT, c->tn, polys, 1, 0, TS, N, 0, TS, N, st);
     if (rc) return rc;
-    return modup_moddown(c, ip_coeff, out, add, add_stride, batch, pq_tmp, nosc, st);
+    return modup_moddown(c, ip_coeff, out, add, add_stride, add_h, batch, pq_tmp, nosc, st);
 }
 
 int kb_modup_qj_to_t(const kbfv_context *c, const uint64_t *x, long xs, uint64_t *out, int batch,
@@ -342,11 +346,11 @@ int kb_modup_t_to_pq(const kbfv_context *c, const uint64_t *in, uint64_t *out, i
 }
 
 int kb_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *out, const uint64_t *add,
-               long add_stride, int batch, hipStream_t st) {
+               long add_stride, int batch, hipStream_t st, int add_h) {
     KB_REQUIRE(c && in && out && batch > 0, "bad modDown arguments");
     KB_REQUIRE(2L * batch <= 65535, "batch too large for one modDown launch");
     hipLaunchKernelGGL(k_moddown, dim3(c->n / KS_BS, c->qn, 2 * batch), dim3(KS_BS), 0, st, c->t, in, out, add,
-                       add_stride, c->pn, c->qn, c->oQ, c->n);
+                       add_stride, add_h, c->pn, c->qn, c->oQ, c->n);
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }

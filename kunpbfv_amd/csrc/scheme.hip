@@ -849,10 +849,8 @@ extern "C" int kbfv_rotate(const kbfv_context *c, const uint64_t *gkey, uint64_t
         KB_TRY(kb_ntt(c, -1, ct + b0 * CTS, w.X, c->oQ, qn, 2, nb, CTS, qn * N, N, CTS, qn * N, N, s));
         KB_TRY(kb_digits_to_t_ntt(c, w.X, CTS, w.CT, nb, nullptr, s));
         KB_TRY(kb_inner_product(c, w.CT, gkey, w.IP, nb, s));
-        KB_TRY(kb_ks_tail(c, w.IP, w.IP, w.MD, nullptr, 0, nb, w.PQ, s));
-        for (int b = 0; b < nb; ++b)  // KS(a) + (0, b): b joins the second polynomial only
-            KB_TRY(kb_poly_binop(c, 0, w.MD + b * CTS + qn * N, w.X + b * CTS + qn * N, w.MD + b * CTS + qn * N,
-                                 c->oQ, qn, 1, s));
+        // KS(a) + (0, b): b joins the second polynomial only
+        KB_TRY(kb_ks_tail(c, w.IP, w.IP, w.MD, w.X, CTS, nb, w.PQ, s, 1));
         KB_TRY(launch_automorphism(c, g, w.MD, w.X, c->oQ, qn, 2 * nb, s));
         KB_TRY(kb_ntt(c, +1, w.X, out + b0 * CTS, c->oQ, qn, 2, nb, CTS, qn * N, N, CTS, qn * N, N, s));
     }

@@ -224,6 +224,16 @@ __device__ __forceinline__ uint64_t kb_fold128(kbfv_u128 v, uint32_t c, uint64_t
     const uint64_t r = kb_mad32((uint32_t)(p >> 28), c, kb_mad32((uint32_t)H, c, L) + w);  // < 2^62
     return kb_csub_sel(kb_ufold(r, c), nq);
 }
+// v below 2^125 modulo a prime 2^60 - c, c < 2^26: the same with the upper word at 2^64,
+// which is 16 c
+__device__ __forceinline__ bool kb_fold125_prime(uint64_t q) { return (q >> 26) == (1ULL << 34) - 1; }
+__device__ __forceinline__ uint64_t kb_fold125(kbfv_u128 v, uint32_t c, uint64_t nq) {
+    const uint32_t c16 = c << 4;                          // below 2^30
+    const uint64_t p = (uint64_t)(uint32_t)(v.hi >> 32) * c16;  // below 2^59
+    const uint64_t w = (uint64_t)((uint32_t)p & 0x0fffffffu) << 32;
+    const uint64_t r = kb_mad32((uint32_t)v.hi, c16, kb_ufold(v.lo, c)) + w;  // below 2^62 + 2^61 + 2^30
+    return kb_csub_sel(kb_ufold(kb_mad32((uint32_t)(p >> 28), c, r), c), nq);
+}
 // signed x, |x| <= 7.9 2^60 -> [0, q)
 __device__ __forceinline__ uint64_t kb_fold_canon(uint64_t x, uint64_t q, uint64_t nq, uint32_t c) {
     return kb_csub_sel(kb_ufold(x + (q << 3), c), nq);

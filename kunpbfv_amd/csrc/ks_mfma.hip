@@ -16,7 +16,8 @@
 // ciphertexts through in tiles of 16: 15 weight passes of MFMAs into biased
 // accumulators (every P_w + 2^22 lies in [0, 2^23]), paired into 32-bit words
 // on the fly, then per output the 128-bit sum rebuilt from its 8 words, the
-// bias removed, and one Barrett reduction.
+// bias removed, and one reduction: folded at bits 60 and 64 where the prime is near
+// 2^60 (28 digits, 128 ciphertexts, n=65536: 8.7 ms, 9.6 with Barrett).
 #include "kbfv_internal.h"
 #include "kbfv_mfma.h"
 #include "kbfv_ops.h"
@@ -80,6 +81,7 @@ __global__ void __launch_bounds__(IM_THREADS, 4)
     const uint32_t tn32 = (uint32_t)TN;  // 8 TN * 16 * 32 fits 31 bits (checked by the launcher)
     const int R2 = 2 * B;
     const uint64_t q = mods[oT + kk], mlo = mus[2 * (oT + kk)], mhi = mus[2 * (oT + kk) + 1];
+    const bool fold = kb_fold125_prime(q);  // uniform
 
     // key layout [2][KD][KB][tn][N] (its first D digits and B blocks are used),
     // row r = h B + b; lane holds rows 16 nt + p16, digits d = 8c + 2g + e
@@ -183,7 +185,8 @@ __global__ void __launch_bounds__(IM_THREADS, 4)
                 const uint64_t lo = a0 + (a1 << 32);
                 uint64_t hi = (a1 >> 32) + a2 + (a3 << 32) + (uint64_t)(lo < a0);
                 hi -= IM_BIAS_HI + (uint64_t)(lo < IM_BIAS_LO);
-                const uint64_t v = kb_barrett128(kbfv_u128{lo - IM_BIAS_LO, hi}, q, mlo, mhi);
+                const kbfv_u128 sum{lo - IM_BIAS_LO, hi};
+                const uint64_t v = fold ? kb_fold125(sum, kb_fold_c(q), 0 - q) : kb_barrett128(sum, q, mlo, mhi);
                 ob[r * IM_OR + p16 * IM_OC + wave] = v;
                 // one output at a time (interleaving them costs registers, not time)
                 __builtin_amdgcn_sched_barrier(0);

@@ -414,7 +414,9 @@ def ntt_alone(stream, polys=256, reps=10):
 
     def fields(p):
         cs, ct, rt, cx, rx = kb.ntt_plan_fields(p, ctx.log_n)
-        return {"plan": hex(p), "passes": 1 if cs == ctx.log_n else 2, "split_log": [cs, ctx.log_n - cs],
+        # the built-in shape's word takes the one-pass kernel for this many limbs
+        one = cs == ctx.log_n or (cs, ct, rt, cx, rx) == kb.ntt_plan_fields(0, ctx.log_n)
+        return {"plan": hex(p), "passes": 1 if one and not p >> 14 else 2, "split_log": [cs, ctx.log_n - cs],
                 "tile_log": [ct, rt]}
 
     res = {"workload": f"negacyclic NTT, N=2^14, {limbs} x 60-bit primes, {polys} polynomials "
@@ -523,12 +525,12 @@ def autotune_report(ctx, tuned):
 
 
 def kernel_roofline(ctx, B, stream):
-    """The dominant kernel, k_ntt_pass, as the pipeline's largest NTT: one
+    """The dominant kernel, the NTT, as the pipeline's largest transform: one
     inverse negacyclic NTT over the QR basis of the 3 tensor polynomials of
     every ciphertext, timed with HIP events on the stream the library launches
     on.  Algorithmic bytes per transform = every limb read once and written
-    once (2 x 512 KiB per 2^16-coefficient limb); a transform is two kernel
-    launches (column and row pass) per chunk of its plan."""
+    once (2 x 512 KiB per 2^16-coefficient limb); a transform is one launch under
+    the built-in plan (k_ntt_reg), else two (column and row pass) per chunk."""
     import torch
     import kunpbfv_amd as kb
     sn = ctx.qn + ctx.rn
@@ -550,16 +552,19 @@ def kernel_roofline(ctx, B, stream):
     plan = ctx.ntt_plan(-1, kb.lib.kbfv_ntt_plan_bucket(limbs))
     chunk = kb.ntt_plan_chunk_bytes(plan)
     chunks = 1 if not chunk else -(-polys // max(1, chunk // (sn * ctx.n * 8)))
-    launches = 2 * chunks
+    one = not chunk and kb.ntt_plan_fields(plan, ctx.log_n) == kb.ntt_plan_fields(0, ctx.log_n)
+    launches = 1 if one else 2 * chunks
     achieved = bytes_per_transform / per_transform_s / 1e9
     traffic, source = NTT_TRAFFIC.get((ctx.log_n, ctx.qn, B, plan), (None, None))
-    return {"kernel": "k_ntt_pass (inverse NTT over the QR basis, whole batch: column + row pass)",
+    name = "k_ntt_reg (inverse NTT over the QR basis, whole batch: one pass)" if one else \
+        "k_ntt_pass (inverse NTT over the QR basis, whole batch: column + row pass)"
+    return {"kernel": name,
             "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": source,
             "unit_of_work": f"one transform of {limbs} limbs of 2^{ctx.log_n} coefficients",
             "bytes_per_transform": bytes_per_transform, "transform_ms": round(per_transform_s * 1e3, 3),
             "launches_per_transform": launches, "avg_launch_ms": round(per_transform_s * 1e3 / launches, 4),
-            "per_pass_frac": round(achieved * 2 / HBM_PEAK_GBS, 4),
+            "per_pass_frac": round(achieved * (1 if one else 2) / HBM_PEAK_GBS, 4),
             "ntt_plan": hex(plan), "chunk_bytes": chunk}
 
 

@@ -406,11 +406,14 @@ __device__ __forceinline__ int xcd_block(int xcd) {
     return (int)blockIdx.x;
 }
 
-// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL;
-// the launch's moduli are all near 2^60 (FOLD) or none is: one kernel for both, with a
-// branch, holds the registers of the larger (a client's round trip on 35-bit primes,
-// n=16384, 64 messages, 393 us against 378)
-template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool FOLD>
+// the moduli of a launch: none near 2^60, all, or some of each.  The kernel for some of
+// each holds the registers of both forms (a client's round trip on 35-bit primes,
+// n=16384, 64 messages, 393 us against 378 with the kernel for none), so it takes mixed
+// launches only.
+enum { SHOUP, FOLD, BOTH };
+
+// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, int KIND>
 __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     k_ntt_pass(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
                const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
@@ -427,9 +430,13 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     bid /= polys;
     const int bi = bid % batch;
     const int l = bid / batch;
-    const uint64_t *in = bi < half ? src + bi * sB : src2 + (bi - half) * sB;
-    pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, false, FOLD>(
-        tile, in + y * sY + l * sL, dst + bi * dB + y * dY + l * dL, tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
+    const uint64_t *in = (bi < half ? src + bi * sB : src2 + (bi - half) * sB) + y * sY + l * sL;
+    uint64_t *out = dst + bi * dB + y * dY + l * dL;
+    if constexpr (KIND == BOTH)
+        pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, in, out, tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
+    else
+        pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, false, KIND == FOLD>(tile, in, out, tw, ninv_tab, w1_tab,
+                                                                                  mods, mod0 + l, grp0);
 }
 
 // A pass for few transforms (the chip is not full and a wave's own chain of
@@ -576,7 +583,14 @@ struct pass_args {
     int half = 0x7fffffff;
 };
 
-template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE>
+// limbs from modulus mod0 on whose primes are all near 2^60 or all not
+int kind_run(const kbfv_context *c, int mod0, int limbs) {
+    int run = 1;
+    while (run < limbs && kb_fold_prime(c->mod[mod0 + run]) == kb_fold_prime(c->mod[mod0])) ++run;
+    return run;
+}
+
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, bool MIXED = false>
 int launch_pass(const pass_args &a) {
     if constexpr (!pass_ok(LOG_N, LOG_S, LOG_T, COLUMN)) {
         kb_set_error("NTT pass 2^%d over tiles of 2^%d is not in the plan space", LOG_S, LOG_T);
@@ -586,17 +600,19 @@ int launch_pass(const pass_args &a) {
         const long groups = (1L << (LOG_N - LOG_S)) / G::C;
         const long blocks = groups * a.limbs * a.polys * a.batch;
         KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
-        const auto go = [&](auto fold) {
-            constexpr bool FOLD = decltype(fold)::value;
-            hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, FOLD>), dim3((unsigned)blocks),
+        const auto go = [&](auto kind) {
+            constexpr int KIND = decltype(kind)::value;
+            hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, KIND>), dim3((unsigned)blocks),
                                dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod,
                                a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd, a.src2,
                                a.half);
         };
-        if (kb_fold_prime(a.c->mod[a.mod0]))
-            go(std::true_type{});
+        if constexpr (MIXED)
+            go(std::integral_constant<int, BOTH>{});
+        else if (kb_fold_prime(a.c->mod[a.mod0]))
+            go(std::integral_constant<int, FOLD>{});
         else
-            go(std::false_type{});
+            go(std::integral_constant<int, SHOUP>{});
         KB_LAUNCH_CHECK();
         return KBFV_OK;
     }
@@ -646,10 +662,14 @@ int small_transform_n(int log_n, int dir, bool noscale, const pass_args &first, 
     }
 }
 
-// pass length 2^log_s (one of three around the default split) and tile 2^log_t
+// pass length 2^log_s (one of three around the default split) and tile 2^log_t; a launch
+// over both kinds of primes takes the built-in shape whatever the plan says (in either pass,
+// so the two fit each other).  One launch per run of a kind took 54 us where one for all
+// takes 16 (inverse, n=32768, 4 polynomials of eight alternating primes)
 template <int LOG_N, bool COLUMN, bool FWD, bool NOSCALE>
 int launch_pass_st(int log_s, int log_t, const pass_args &a) {
     constexpr int s0 = (COLUMN ? col_log_default(LOG_N) : LOG_N - col_log_default(LOG_N)) - 1;
+    if (kind_run(a.c, a.mod0, a.limbs) < a.limbs) return launch_pass<LOG_N, s0 + 1, 12, COLUMN, FWD, NOSCALE, true>(a);
 #define KB_NTT_ST(DS, LT)                                                   \
     if (log_s == s0 + DS && log_t == LT) return launch_pass<LOG_N, s0 + DS, LT, COLUMN, FWD, NOSCALE>(a);
     KB_NTT_ST(0, 11) KB_NTT_ST(0, 12) KB_NTT_ST(0, 13)
@@ -861,6 +881,20 @@ bool one_pass(int log_n, long rows) {
     return 100 * rows >= (log_n == 15 ? 57 : 80) * held;
 }
 
+// Whether a launch over both kinds of primes goes run by run.  The one-pass kernel saves
+// about 2.5 ps a word on the primes near 2^60, another run costs about 8 us.  All in one /
+// run by run, inverse, in us: seven near 2^60 and one of 45 bits, 64 polynomials, N=2^13
+// 38/36, 2^14 63/55, 2^15 133/118, 256 at 2^14 266/184; 60, six of 45 and 60 bits,
+// 2^14 64 polynomials 64/85, 2^15 256 563/526; eight alternating, 2^14 64 polynomials 63/137.
+bool split_kinds(const kbfv_context *c, int mod0, int limbs, long transforms) {
+    long near = 0, runs = 0;
+    for (int l = 0, run; l < limbs; l += run, ++runs) {
+        run = kind_run(c, mod0 + l, limbs - l);
+        if (kb_fold_prime(c->mod[mod0 + l])) near += run;
+    }
+    return (near * transforms << c->log_n) >= (runs - 1) << 22;
+}
+
 int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, const uint64_t *src, uint64_t *dst,
                   int mod0, int limbs, int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL,
                   hipStream_t st, const uint64_t *src2 = nullptr) {
@@ -872,18 +906,16 @@ int ntt_with_plan(const kbfv_context *c, int dir, bool noscale, uint32_t plan, c
         const pass_args second{c, dst, dst, mod0, limbs, polys, batch, dB, dY, dL, dB, dY, dL, 0, st};
         return small_transform_n(c->log_n, dir, noscale, first, second);
     }
-    // one kind of prime per launch below
-    const bool near60 = kb_fold_prime(c->mod[mod0]);
-    int run = 1;
-    while (run < limbs && kb_fold_prime(c->mod[mod0 + run]) == near60) ++run;
-    if (run < limbs) {
+    const int run = kind_run(c, mod0, limbs);
+    const bool mixed = run < limbs, near60 = !mixed && kb_fold_prime(c->mod[mod0]);
+    if (mixed && split_kinds(c, mod0, limbs, (long)polys * batch)) {
         KB_TRY(ntt_with_plan(c, dir, noscale, plan, src, dst, mod0, run, polys, batch, sB, sY, sL, dB, dY, dL, st, src2));
         return ntt_with_plan(c, dir, noscale, plan, src + run * sL, dst + run * dL, mod0 + run, limbs - run, polys, batch,
                              sB, sY, sL, dB, dY, dL, st, src2 ? src2 + run * sL : nullptr);
     }
     if (near60 && (plan == 0 ? one_pass(c->log_n, (long)limbs * polys * batch) : single_pass(c->log_n, f)))
         return kb_ntt_reg(c, dir, noscale, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, st, src2, half);
-    if (single_pass(c->log_n, f)) {
+    if (single_pass(c->log_n, f) && !mixed) {
         const pass_args a{c, src, dst, mod0, limbs, polys, batch, sB, sY, sL, dB, dY, dL, f.col_x, st, src2, half};
         if (dir > 0) return launch_limb_n<true, false>(a);
         return noscale ? launch_limb_n<false, true>(a) : launch_limb_n<false, false>(a);

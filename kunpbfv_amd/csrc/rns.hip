@@ -287,6 +287,15 @@ int kb_poly_binop(const kbfv_context *c, int op, const uint64_t *a, const uint64
     return KBFV_OK;
 }
 
+// Whether a launch is too small for the matrix kernel, whose workgroups first read 64 KB of
+// matrix each: matrix / register kernel, Q -> R at N=4096 in us: 13 primes, 16
+// polynomials 9.0/8.1, 32 10.1/12.1; 20 primes, 8 14.2/9.8, 16 14.9/14.7 (a product of 4
+// ciphertexts of 16 primes 184/191), 32 17.4/23.6; 28 primes, 4 17.0/10.7, 8 17.4/15.1,
+// 16 18.5/21.2
+static bool few_coefficients(const kbfv_context *c, int polys) {
+    return c->t.cv_qr && ((long)polys << c->log_n) <= (c->qn <= 14 ? 1L << 16 : 1L << 15);
+}
+
 int kb_bconv(const kbfv_context *c, bool q_to_r, const uint64_t *x, long in_stride, uint64_t *y,
              long out_stride, int polys, hipStream_t st, bool noscale) {
     KB_REQUIRE(c && x && y && polys > 0, "bad bconv arguments");
@@ -294,7 +303,7 @@ int kb_bconv(const kbfv_context *c, bool q_to_r, const uint64_t *x, long in_stri
     KB_REQUIRE(q_to_r || !noscale, "unscaled input only for Q -> R");
     // the matrix cores for long chains, one coefficient per thread up to 31 limbs,
     // the LDS kernel below for longer ones
-    if (c->t.mx_qr) return kb_bconv_mfma(c, q_to_r, x, in_stride, y, out_stride, polys, st, noscale);
+    if (c->t.mx_qr && !few_coefficients(c, polys)) return kb_bconv_mfma(c, q_to_r, x, in_stride, y, out_stride, polys, st, noscale);
     if (c->t.cv_qr) return kb_bconv_reg(c, q_to_r, x, in_stride, y, out_stride, polys, st, noscale);
     const int tiles = c->n / BC_TILE;
     const kb_dev_tables &t = c->t;
@@ -335,7 +344,7 @@ int kb_tensor(const kbfv_context *c, const uint64_t *ct1, const uint64_t *ct2, u
 int kb_scale_round(const kbfv_context *c, const uint64_t *x, uint64_t *y, int polys, hipStream_t st) {
     KB_REQUIRE(c && x && y && polys > 0, "bad scale-round arguments");
     KB_REQUIRE(c->qn <= BC_MAXIN, "too many limbs for scale-and-round");
-    if (c->t.mx_sr) return kb_scale_round_mfma(c, x, y, polys, st);
+    if (c->t.mx_sr && !few_coefficients(c, polys)) return kb_scale_round_mfma(c, x, y, polys, st);
     if (c->t.cv_sr) return kb_scale_round_reg(c, x, y, polys, st);
     const int tiles = c->n / BC_TILE;
     hipLaunchKernelGGL(k_scale_round, dim3(tiles * polys), dim3(BC_TILE * BC_WAVES), 0, st, c->t, x, y,

@@ -37,11 +37,13 @@
 
 namespace {
 
+// blockIdx.y: outputs j0 = per blockIdx.y .. of the thread's coefficient
 template <int IN, bool SR>
 __global__ void __launch_bounds__(256)
     k_rns_conv(const uint64_t *__restrict__ x, long in_stride, uint64_t *__restrict__ y, long out_stride,
                const uint64_t *__restrict__ tab, const kb_conv_in *__restrict__ inp,
-               const double *__restrict__ est, int out_n, int log_n, int log_bs) {
+               const double *__restrict__ est, int out_n, int per, int log_n, int log_bs) {
+    const int j0 = (int)blockIdx.y * per, j1 = min(j0 + per, out_n);
     const long n = 1L << log_n;
     const long poly = blockIdx.x >> (log_n - log_bs);
     const long k = (long)((blockIdx.x & ((1 << (log_n - log_bs)) - 1)) << log_bs) + threadIdx.x;
@@ -68,15 +70,15 @@ __global__ void __launch_bounds__(256)
 
     constexpr int RW = kb_conv_row_words(IN);
     constexpr int G = 15, NG = (IN + G - 1) / G;  // rows per middle accumulator, their number
-    uint64_t diag = SR ? xp[IN * n] : 0;
+    uint64_t diag = SR ? xp[(IN + j0) * n] : 0;
 #pragma unroll 1
-    for (int j = 0; j < out_n; ++j) {
+    for (int j = j0; j < j1; ++j) {
         const uint64_t *row = tab + (long)j * RW;
         const int *m = (const int *)row;
 #pragma unroll
         for (int i = 0; i < IN; ++i) kb_pin(x0[i]), kb_pin(x1[i]), kb_pin(xs[i]);
         uint64_t dnext = 0;
-        if (SR) dnext = xp[(IN + min(j + 1, out_n - 1)) * n];
+        if (SR) dnext = xp[(IN + min(j + 1, j1 - 1)) * n];
         int64_t lo = 0, hi = 0, mid[NG];
         uint64_t outer = 0;  // lo + hi of the groups before
 #pragma unroll
@@ -130,45 +132,64 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+struct conv_args {
+    const uint64_t *x;
+    long in_stride;
+    uint64_t *y;
+    long out_stride;
+    const uint64_t *tab;
+    const kb_conv_in *inp;
+    const double *est;
+    int in_n, out_n, polys, log_n;
+    hipStream_t st;
+};
+
 template <bool SR, int IN = 1>
-int launch(int in_n, unsigned blocks, int bs, hipStream_t st, const uint64_t *x, long in_stride, uint64_t *y,
-           long out_stride, const uint64_t *tab, const kb_conv_in *inp, const double *est, int out_n, int log_n, int log_bs) {
+int launch(const conv_args &a, dim3 grid, int per, int log_bs) {
     if constexpr (IN <= KB_CONV_MAXROWS - (SR ? 1 : 0)) {
-        if (in_n != IN)
-            return launch<SR, IN + 1>(in_n, blocks, bs, st, x, in_stride, y, out_stride, tab, inp, est, out_n, log_n,
-                                      log_bs);
-        hipLaunchKernelGGL((k_rns_conv<IN, SR>), dim3(blocks), dim3(bs), 0, st, x, in_stride, y, out_stride, tab, inp,
-                           est, out_n, log_n, log_bs);
+        if (a.in_n != IN) return launch<SR, IN + 1>(a, grid, per, log_bs);
+        hipLaunchKernelGGL((k_rns_conv<IN, SR>), grid, dim3(1 << log_bs), 0, a.st, a.x, a.in_stride, a.y, a.out_stride,
+                           a.tab, a.inp, a.est, a.out_n, per, a.log_n, log_bs);
         KB_LAUNCH_CHECK();
         return KBFV_OK;
     } else {
-        kb_set_error("RNS conversion of %d limbs exceeds the register kernel", in_n);
+        kb_set_error("RNS conversion of %d limbs exceeds the register kernel", a.in_n);
         return KBFV_EINVAL;
     }
 }
 
-// workgroups of one wave while that leaves compute units idle, of four otherwise
-int log_block(long coeffs) { return coeffs < 256L * 1024 ? 6 : 8; }
+// Workgroups of one wave while that leaves compute units idle, of four otherwise.
+// Where even single waves leave SIMDs idle, a coefficient's outputs are split over up
+// to eight threads that each repeat the input part (about the work of two outputs):
+// 28 primes, N=4096, Q -> R of 1 / 4 / 8 polynomials 26.5 / 26.9 / 29.8 us whole, 8.0 /
+// 12.5 / 15.1 in 8 / 4 / 4 parts; 12 primes, 16 polynomials 11.0 whole, 8.0 in two, 32
+// polynomials 11.0 whole, 11.5 in two; 30 primes of 45 bits, 32 polynomials 60 whole,
+// 44 in two, 64 polynomials 67 whole, 78 in two.  Chains of up to 8 primes take the 7.3
+// us of an empty call either way.
+template <bool SR>
+int launch_any(const conv_args &a) {
+    const long coeffs = (long)a.polys << a.log_n, waves = coeffs / 64;
+    const int lb = coeffs < 256L * 1024 ? 6 : 8;
+    const long blocks = (long)a.polys << (a.log_n - lb);
+    KB_REQUIRE(blocks < (1L << 31), "grid too large");
+    int parts = 1;
+    if (a.in_n > 8) parts = (int)std::min(8L, std::max(1L, (a.in_n > 16 && waves > 1024 ? 4096 : 2048) / waves));
+    const int per = (a.out_n + parts - 1) / parts;
+    return launch<SR>(a, dim3((unsigned)blocks, (a.out_n + per - 1) / per), per, lb);
+}
 
 }  // namespace
 
 int kb_bconv_reg(const kbfv_context *c, bool q_to_r, const uint64_t *x, long in_stride, uint64_t *y, long out_stride,
                  int polys, hipStream_t st, bool noscale) {
-    const int in_n = q_to_r ? c->qn : c->rn, out_n = q_to_r ? c->rn : c->qn;
     const kb_dev_tables &t = c->t;
-    const int lb = log_block((long)polys * c->n);
-    const long blocks = (long)polys * (c->n >> lb);
-    KB_REQUIRE(blocks < (1L << 31), "grid too large");
-    return launch<false>(in_n, (unsigned)blocks, 1 << lb, st, x, in_stride, y, out_stride, q_to_r ? t.cv_qr : t.cv_rq,
-                         q_to_r ? (noscale ? t.cv_in_qn : t.cv_in_q) : t.cv_in_r, q_to_r ? t.q_inv : t.r_inv, out_n,
-                         c->log_n, lb);
+    return launch_any<false>({x, in_stride, y, out_stride, q_to_r ? t.cv_qr : t.cv_rq,
+                              q_to_r ? (noscale ? t.cv_in_qn : t.cv_in_q) : t.cv_in_r, q_to_r ? t.q_inv : t.r_inv,
+                              q_to_r ? c->qn : c->rn, q_to_r ? c->rn : c->qn, polys, c->log_n, st});
 }
 
 int kb_scale_round_reg(const kbfv_context *c, const uint64_t *x, uint64_t *y, int polys, hipStream_t st) {
     const kb_dev_tables &t = c->t;
-    const int lb = log_block((long)polys * c->n);
-    const long blocks = (long)polys * (c->n >> lb);
-    KB_REQUIRE(blocks < (1L << 31), "grid too large");
-    return launch<true>(c->qn, (unsigned)blocks, 1 << lb, st, x, (long)(c->qn + c->rn) * c->n, y, (long)c->rn * c->n,
-                        t.cv_sr, nullptr, t.sr_frac, c->rn, c->log_n, lb);
+    return launch_any<true>({x, (long)(c->qn + c->rn) * c->n, y, (long)c->rn * c->n, t.cv_sr, nullptr, t.sr_frac, c->qn,
+                             c->rn, polys, c->log_n, st});
 }

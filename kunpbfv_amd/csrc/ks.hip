@@ -324,11 +324,16 @@ int kb_modup_pq_to_t(const kbfv_context *c, const uint64_t *x, uint64_t *out, in
 int kb_inner_product(const kbfv_context *c, const uint64_t *cin, const uint64_t *key, uint64_t *out,
                      int batch, hipStream_t st) {
     KB_REQUIRE(c && cin && key && out && batch > 0, "bad inner-product arguments");
-    // the matrix cores pay for long keys and large batches only: 28 digits at N =
-    // 2^16, 40 ciphertexts 4.37 against 4.16 ms, 48 4.45 against 4.94, 128 9.32
-    // against 12.7; 18 digits, 48 ciphertexts 3.25 against 3.71 ms; 13 digits, 64
-    // ciphertexts at N = 2^15 1.22 against 0.73 ms
-    if (c->dnum > 16 && batch >= 44) {
+    // The matrix cores pay for long keys and column tiles of 16 ciphertexts that are well
+    // filled; their time is a part for the key and one per tile, the holding kernel's
+    // goes by the ciphertext.  Matrix / holding kernel, us: 17 digits at N=2^14, 16
+    // ciphertexts 279/323, 17 427/350, 24 446/460, 32 446/599, 33 573/634, 48 629/882;
+    // 24 digits at 2^15, 16 815/758, 24 1164/1071, 28 1157/1235, 33 1488/1448, 40
+    // 1490/1686; 28 digits at 2^16, 32 3291/3206, 40 3989/3939, 44 4028/4297, 64
+    // 4968/6118; 13 digits, 64 ciphertexts at 2^15 1220/730
+    const int tiles16 = (batch + 15) / 16;
+    const int least = (c->dnum <= 20 ? 6 : 8) + 9 * tiles16 + (c->log_n > 15 ? 7 : 0);
+    if (c->dnum > 16 && batch >= least) {
         const int r = kb_inner_product_mfma(c, cin, key, out, batch, st);
         if (r != 1) return r;
     }

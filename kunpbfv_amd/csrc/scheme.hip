@@ -1018,12 +1018,20 @@ extern "C" int kbfv_external_product(const kbfv_context *c, const uint64_t *rgsw
     uint64_t *coef = bp.take(2 * L * batch), *dig = bp.take(8 * L * batch);
     hipStream_t s = S(st);
     KB_TRY(kb_ntt(c, -1, ct, coef, c->oQ, qn, 2, batch, 2 * L, L, N, 2 * L, L, N, s));
-    // the auxiliary basis costs a basis change of the whole RGSW ciphertext, which
-    // enough ciphertexts have to share: 28 primes at N = 2^16, 8 ciphertexts 31.6 against
-    // 27.5 ms, 12 31.5 against 40.6; 13 at 2^15, 12 4.56 against 4.60, 16 4.77 against
-    // 6.03; 6 at 2^14, 16 0.80 against 0.78, 32 0.95 against 1.53; 2 at 2^13, 64 0.37
-    // against 0.48
-    const int np = batch >= 12 && batch * qn >= 100 ? kb_ext_aux_primes(c, rows, base_bits) : 0;
+    // The auxiliary basis costs a basis change of the whole RGSW ciphertext, which enough
+    // ciphertexts have to share, fewer the more words one polynomial has to keep the chip
+    // busy with.  General / auxiliary path, base 2^20, us: N=2^16, 28 primes, 8
+    // ciphertexts 27500/31600, 12 40600/31500; 12 of 50 bits, 11 ciphertexts 6900/6800, 12
+    // 7524/7001; 9 primes, 12 3901/4370, 13 4285/4323, 14 4640/4332; 2^15, 13 primes, 12
+    // 4224/4351, 13 4612/4228; 9 primes, 14 2386/2528, 15 2568/2371; 2^14, 12 primes, 16
+    // 2247/2379, 17 2470/2239; 2^13, 8 of 45 bits, 17 777/831, 20 886/705; 2^12, 4 primes, 16
+    // 251/266, 20 305/234.  Short chains gain less, as a digit has as many transforms there
+    // as here: 4 primes at 2^16, 25 1653/1644; 3 there, 64 2625/2812; 2 at 2^15, 100
+    // 1395/1514, at 2^14, 50 432/407; 1 at 2^14, 200 691/815, at 2^13, 128 399/386, 100 320/340.
+    const int least = L >= 3L << 18 ? 12 : L >= 3L << 17 ? 13 : L >= 7L << 15 ? 15 : L >= 5L << 15 || qn > 16 ? 17 : 18;
+    const bool enough = batch >= least && batch * (long)qn >= (qn == 1 && c->log_n > 12 ? 112 : 100) &&
+                        qn >= c->log_n - 12;
+    const int np = enough ? kb_ext_aux_primes(c, rows, base_bits) : 0;
     if (np && kb_ext_aux_rows(c, batch, np) >= 1)
         return kb_external_product_aux(c, rgsw, coef, out, dig, batch, rows, nd, base_bits, np, s);
     KB_TRY(fill_zero(out, 2 * L * batch, s));

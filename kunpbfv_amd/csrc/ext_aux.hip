@@ -536,15 +536,18 @@ int run(const kbfv_context *c, const uint64_t *rgsw, const uint64_t *coef, uint6
     }
     const lay32 al{(int)hls, np * hls * N, 64, hls * N, hls * 64};
     KB_TRY(A::inverse(c, acc, al, (int)(batch * hls), np, st));
-    KB_REQUIRE(batch <= 65535, "batch too large for one launch");
-    const dim3 grid((unsigned)(N / 256), (unsigned)hls, (unsigned)batch);
-    if (np == 3)
-        hipLaunchKernelGGL(k32_lift<3>, grid, dim3(256), 0, st, acc, out, c->t.aux_mod, c->t.aux_mix, c->t.aux_lift,
-                           c->qn, (int)hls, c->log_n);
-    else
-        hipLaunchKernelGGL(k32_lift<4>, grid, dim3(256), 0, st, acc, out, c->t.aux_mod, c->t.aux_mix, c->t.aux_lift,
-                           c->qn, (int)hls, c->log_n);
-    KB_LAUNCH_CHECK();
+    for (int b0 = 0; b0 < batch; b0 += 65535) {  // grid z
+        const dim3 grid((unsigned)(N / 256), (unsigned)hls, (unsigned)std::min(batch - b0, 65535));
+        const uint32_t *a = acc + hls * np * b0 * N;
+        uint64_t *o = out + hls * b0 * N;
+        if (np == 3)
+            hipLaunchKernelGGL(k32_lift<3>, grid, dim3(256), 0, st, a, o, c->t.aux_mod, c->t.aux_mix, c->t.aux_lift,
+                               c->qn, (int)hls, c->log_n);
+        else
+            hipLaunchKernelGGL(k32_lift<4>, grid, dim3(256), 0, st, a, o, c->t.aux_mod, c->t.aux_mix, c->t.aux_lift,
+                               c->qn, (int)hls, c->log_n);
+        KB_LAUNCH_CHECK();
+    }
     return kb_ntt_inplace(c, +1, out, c->oQ, c->qn, 2 * batch, st);
 }
 

@@ -4,9 +4,9 @@
 // modUpQjtoT_23_kernel (:86-135), external_product_T_kernel and its
 // _swk_reuse variant (include/ExternalProduct.cuh:11-177), modUpTtoPQl_23_kernel
 // (include/BasisConv.cuh:159-213) and the modDownPQltoQl_23 kernels (:233-298).
-// The float overflow estimates (`vv += (float)x / (float)m`, truncation, and
-// the 128-bit wrap of `acc - vv * (M mod m)`) are kept operation for operation;
-// the surrounding arithmetic is exact with canonical outputs.
+// The float overflow estimates (`vv += (float)x / (float)m`, truncation) are kept
+// operation for operation, but for what overflow_count says; the surrounding
+// arithmetic is exact with canonical outputs.
 //
 // MI355X design: with one special prime (K = 1) the digit decomposition of a
 // limb is the limb itself, so "modUp Qj -> T then NTT over T" is one NTT that
@@ -20,6 +20,12 @@ constexpr int KS_BS = 256;
 constexpr int KS_MAXG = 16;  // max gamma / tn held in registers
 
 inline unsigned blocks_for(long total, int bs) { return (unsigned)((total + bs - 1) / bs); }
+
+// Overflow count of a block of cnt primes from the float estimate of its sum.  The
+// estimate is one too large for the top 2^-25 of the residues: with one prime there is
+// no overflow; with several the callers subtract modulo each T prime, so that the digit
+// stays a representative of its residues (a 128-bit difference would wrap).
+__device__ __forceinline__ int overflow_count(float vv, int cnt) { return cnt > 1 ? (int)vv : 0; }
 
 // x: [batch][qn][N] -> out: [batch][dnum][tn][N]
 __global__ void k_modup_qj_to_t(kb_dev_tables t, const uint64_t *__restrict__ x, long xs,
@@ -43,13 +49,13 @@ __global__ void k_modup_qj_to_t(kb_dev_tables t, const uint64_t *__restrict__ x,
         const float rr = (float)rb[j];
         vv += rr / (float)q;
     }
-    const int vf = (int)vv;
+    const int vf = overflow_count(vv, cnt);
     uint64_t *op = out + (bt * dnum + b) * (long)tn * n + k;
     for (int kk = 0; kk < tn; ++kk) {
         const int m = oT + kk;
         kbfv_u128 acc{0, 0};
         for (int j = 0; j < cnt; ++j) kb_mac128(acc, rb[j], t.qj_hat_mod_t[(b * tn + kk) * pn + j]);
-        kb_sub128(acc, (uint64_t)vf * t.qj_mod_t[b * tn + kk]);
+        kb_mac128(acc, vf, t.mod[m] - t.qj_mod_t[b * tn + kk]);
         op[(long)kk * n] = kb_barrett128(acc, t.mod[m], t.mu[2 * m], t.mu[2 * m + 1]);
     }
 }
@@ -75,13 +81,13 @@ __global__ void k_modup_pq_to_t(kb_dev_tables t, const uint64_t *__restrict__ x,
         rb[j] = kb_shoup(xp[(long)idx * n], h.w, h.ws, r);
         vv += (float)rb[j] / (float)r;
     }
-    const int vf = (int)vv;
+    const int vf = overflow_count(vv, cnt);
     uint64_t *op = out + (bt * B + b) * (long)tn * n + k;
     for (int kk = 0; kk < tn; ++kk) {
         const int m = oT + kk;
         kbfv_u128 acc{0, 0};
         for (int j = 0; j < cnt; ++j) kb_mac128(acc, rb[j], t.ri_hat_mod_t[(b * tn + kk) * gamma + j]);
-        kb_sub128(acc, (uint64_t)vf * t.ri_mod_t[kk * B + b]);
+        kb_mac128(acc, vf, t.mod[m] - t.ri_mod_t[kk * B + b]);
         op[(long)kk * n] = kb_barrett128(acc, t.mod[m], t.mu[2 * m], t.mu[2 * m + 1]);
     }
 }

@@ -11,8 +11,13 @@
  *   modUpTtoPQl_23_kernel         include/BasisConv.cuh:159-213
  *   modDownPQltoQl_23_*_kernel    include/BasisConv.cuh:233-298 (host :300-317)
  * with the float overflow estimate `vv += (float)x / (float)m`, `(int)vv`
- * and the 128-bit wrap-around of `acc - vv_floor * (M mod m)` restated
- * exactly.
+ * restated exactly.  In Q_j->T and PQ->T the estimate is one too large for the
+ * top residues of a block (about 2^-25 of them).  A block of one prime has no
+ * overflow and takes none here; for several, M times the count is subtracted
+ * modulo each t_k (the reference subtracts in 128 bits, which wraps round and
+ * adds 2^128 where the count exceeds the sum: such a digit or key coefficient
+ * is no representative of its residues, and products made with it do not
+ * decrypt).
  *
  * Pinned by (tests/test_oracle_ks.py), Python big integers: Q_j->T and PQ->T
  * equal the CRT value of the block residues in [0, Q_j) / [0, R_b) reduced mod
@@ -37,12 +42,13 @@
 static uint64_t reduce128(u128 a, uint64_t m) { return (uint64_t)(a % m); }
 
 /* The Q_j -> T and PQ -> T conversions truncate the float overflow estimate
- * (`(int)vv`, include/BasisConv.cuh:32,112). */
+ * (`(int)vv`, include/BasisConv.cuh:32,112); the sum of a block of one prime is
+ * below 1 whatever its float quotient rounds to. */
 #if OR_MUTATION == 2 /* planted mistake (tests only): the estimate rounded */
 #include <math.h>
-#define TRUNC_VV(v) ((int)lrintf(v))
+#define OVERFLOW_COUNT(v, cnt) ((int)lrintf(v))
 #else
-#define TRUNC_VV(v) ((int)(v))
+#define OVERFLOW_COUNT(v, cnt) ((cnt) > 1 ? (int)(v) : 0)
 #endif
 
 /* x_q: [qn][N] coefficient form -> out_t: [dnum][tn][N] */
@@ -61,12 +67,12 @@ void or_modup_qj_to_t(const or_ctx *c, const uint64_t *x_q, uint64_t *out_t) {
                 float rr = (float)rb[j];
                 vv += rr / (float)qi;
             }
-            int vf = TRUNC_VV(vv);
+            int vf = OVERFLOW_COUNT(vv, cnt);
             for (int i = 0; i < tn; i++) {
                 uint64_t t = c->mod[c->oT + i];
                 u128 acc = 0;
                 for (int j = 0; j < cnt; j++) acc += (u128)rb[j] * c->qj_hat_mod_t[(b * tn + i) * pn + j];
-                acc -= (u128)(uint64_t)((uint64_t)vf * c->qj_mod_t[b * tn + i]);
+                acc += (u128)(uint64_t)vf * (t - c->qj_mod_t[b * tn + i]);
                 out_t[((size_t)b * tn + i) * N + k] = reduce128(acc, t);
             }
         }
@@ -87,12 +93,12 @@ void or_modup_pq_to_t(const or_ctx *c, const uint64_t *x_pq, uint64_t *out_t) {
                 rb[j] = or_mulmod(x_pq[(size_t)(b * g + j) * N + k], c->ri_hatinv[b * g + j], ri);
                 vv += (float)rb[j] / (float)ri;
             }
-            int vf = TRUNC_VV(vv);
+            int vf = OVERFLOW_COUNT(vv, cnt);
             for (int i = 0; i < tn; i++) {
                 uint64_t t = c->mod[c->oT + i];
                 u128 acc = 0;
                 for (int j = 0; j < cnt; j++) acc += (u128)rb[j] * c->ri_hat_mod_t[(b * tn + i) * g + j];
-                acc -= (u128)(uint64_t)((uint64_t)vf * c->ri_mod_t[i * c->ri_blocks + b]);
+                acc += (u128)(uint64_t)vf * (t - c->ri_mod_t[i * c->ri_blocks + b]);
                 out_t[((size_t)b * tn + i) * N + k] = reduce128(acc, t);
             }
         }

@@ -19,11 +19,11 @@
 // accumulators and no carry.  The matrix comes through the scalar cache.  |x0 m0|
 // and |x1 m1| are at most 2^58 and the middle product at most 2^59: 31 rows
 // fit the outer accumulators, 15 the middle one, which is closed after every
-// 15 rows (the third product may wrap: only middle = third - first - second
-// has to fit).  Carrying the middle upwards gives the sum as f 2^60 + L with
-// L in [0, 2^60); for 2^(s-1) < p < 2^s its quotient H by 2^s fits 63 bits and a
-// sign, and the result is [(H + 2^63) (2^s mod p) + (L mod 2^s) + const]_p,
-// one Shoup product and three conditional subtractions.
+// 15 full rows, scale-and-round's diagonal among them (the third product may wrap: only
+// middle = third - first - second has to fit).  Carrying the middle upwards gives the
+// sum as f 2^60 + L with L in [0, 2^60); for 2^(s-1) < p < 2^s its quotient H by 2^s fits
+// 63 bits and a sign, and the result is [(H + 2^63) (2^s mod p) + (L mod 2^s) +
+// const]_p, one Shoup product and three conditional subtractions.
 //
 // Bound by VALU issue: a multiply-add takes 5.2 cycles of a SIMD, any other
 // multiply 4.4, an output about 30 of them besides its rows.  2 primes, 36
@@ -69,7 +69,10 @@ __global__ void __launch_bounds__(256)
     const uint64_t nu = SR ? kb_f64_to_u64_sat(acc) : 0;
 
     constexpr int RW = kb_conv_row_words(IN);
-    constexpr int G = 15, NG = (IN + G - 1) / G;  // rows per middle accumulator, their number
+    // rows of full size (scale-and-round's diagonal is one, alpha's row is small) per middle
+    // accumulator, and the number of accumulators
+    constexpr int G = 15, NG = (IN + (SR ? 1 : 0) + G - 1) / G;
+    static_assert(NG * G >= IN + (SR ? 1 : 0), "a middle accumulator holds 15 full rows");
     uint64_t diag = SR ? xp[(IN + j0) * n] : 0;
 #pragma unroll 1
     for (int j = j0; j < j1; ++j) {

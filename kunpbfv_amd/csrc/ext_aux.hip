@@ -199,7 +199,7 @@ __device__ __forceinline__ void rows_in(uint32_t *tile, const uint32_t *__restri
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = (threadIdx.x + j * G::T) * 4;
-        const uint4 v = *(const uint4 *)(g + lay.at(e));
+        const kb_u32x4 v = *(const kb_u32x4 *)(g + lay.at(e));
         uint32_t *t = tile + e + (e >> 4);
         t[0] = v.x, t[1] = v.y, t[2] = v.z, t[3] = v.w;
     }
@@ -233,7 +233,7 @@ __global__ void __launch_bounds__((Geo32<LOG_N, false>::T))
         uint32_t v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = canon32(t[i], md.one_s, md.p);
-        *(uint4 *)(g + lay.at(e)) = make_uint4(v[0], v[1], v[2], v[3]);
+        *(kb_u32x4 *)(g + lay.at(e)) = kb_u32x4{v[0], v[1], v[2], v[3]};
     }
 }
 
@@ -262,7 +262,7 @@ __global__ void __launch_bounds__((Geo32<LOG_N, false>::T))
     for (int j = 0; j < 4; ++j) {
         const int e = (threadIdx.x + j * G::T) * 4;
         const uint32_t *t = tile + e + (e >> 4);
-        *(uint4 *)(g + lay.at(e)) = make_uint4(t[0], t[1], t[2], t[3]);
+        *(kb_u32x4 *)(g + lay.at(e)) = kb_u32x4{t[0], t[1], t[2], t[3]};
     }
 }
 
@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(64 * AM_MAXW)
             const kb_aux_mod *__restrict__ mods, int np, int hls, int rc, int first, int log_n, int batch) {
     constexpr int PF = (AM_CT * MAXR + 4 * AM_MINW - 1) / (4 * AM_MINW);
     constexpr int ROWS = AM_CT * MAXR + 4;
-    __shared__ uint32_t xs[2][ROWS][64];
+    __shared__ alignas(16) uint32_t xs[2][ROWS][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int waves = blockDim.x >> 6;
@@ -340,7 +340,7 @@ __global__ void __launch_bounds__(64 * AM_MAXW)
         for (int u = 0; u < PF; ++u) {
             const int j = min(jl + 4 * waves * u, AM_CT * rc - 1);
             const int c = j >= rc ? 1 : 0;
-            pf[u] = *(const u32x4 *)(src + (long)min(ct + c, batch - 1) * rc * cts + (j - (c ? rc : 0)) * 64);
+            pf[u] = *(const kb_u32x4 *)(src + (long)min(ct + c, batch - 1) * rc * cts + (j - (c ? rc : 0)) * 64);
         }
     };
     auto commit = [&](int buf) {

@@ -17,6 +17,10 @@ struct kbfv_u128 {
     uint64_t lo, hi;
 };
 
+// 16 bytes of a caller's buffer, which need be aligned to its 8-byte words only
+typedef uint64_t kb_u64x2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef uint32_t kb_u32x4 __attribute__((ext_vector_type(4), aligned(8)));
+
 __device__ __forceinline__ uint64_t kb_mulhi(uint64_t a, uint64_t b) { return __umul64hi(a, b); }
 
 // a mod q for a in [0, 2q)

@@ -32,7 +32,7 @@ __device__ __forceinline__ void load_v(const uint64_t *p, uint64_t (&o)[V]) {
     if constexpr (V == 1) {
         o[0] = *p;
     } else {
-        const ulong2 v = *(const ulong2 *)p;
+        const kb_u64x2 v = *(const kb_u64x2 *)p;
         o[0] = v.x, o[1] = v.y;
     }
 }
@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(64 * IS_WAVES)
                 if constexpr (V == 1)
                     *op = o[0];
                 else
-                    *(ulong2 *)op = make_ulong2(o[0], o[1]);
+                    *(kb_u64x2 *)op = kb_u64x2{o[0], o[1]};
             }
         }
     }

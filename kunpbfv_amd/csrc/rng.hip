@@ -138,7 +138,6 @@ __global__ void k_sample(kb_dev_tables t, kb_stream_key key, uint64_t entry0,
 // with a stride between lanes: 24 messages of 6 limbs, n=16384, 64 + 2 x 22 us and 29
 // for Delta m and its sum against 21.  grid (n / 512, batch)
 constexpr int ENC_RUN = 512;
-typedef uint64_t word2 __attribute__((ext_vector_type(2), aligned(8)));  // scratch need not be 16-byte aligned
 __global__ void __launch_bounds__(192)
     k_enc_sample(kb_dev_tables t, kb_stream_key kv, kb_stream_key k0, kb_stream_key k1, const uint64_t *__restrict__ m,
                  uint64_t *__restrict__ out, uint64_t plain, uint64_t negq, uint64_t negq_s, int qn, int oQ, int n,
@@ -180,14 +179,14 @@ __global__ void __launch_bounds__(192)
 #pragma unroll
         for (int i = 0; i < ENC_RUN / 128; ++i) {
             const int k = i * 128 + lane * 2;
-            word2 v;
+            kb_u64x2 v;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int x = smp[which][k + j];
                 v[j] = x < 0 ? q - (uint64_t)(-x) : (uint64_t)x;
                 if (which == 2) v[j] = kb_addmod(v[j], kb_shoup(mq[k + j], ti.w, ti.ws, q), q);
             }
-            *(word2 *)(o + k) = v;
+            *(kb_u64x2 *)(o + k) = v;
         }
     }
 }

@@ -388,9 +388,9 @@ template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, 
 __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
                                           const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
                                           const kbfv_tw *__restrict__ w1_tab, const uint64_t *__restrict__ mods,
-                                          const int m, const int grp0, const int dshift = 0,
+                                          const int m, const int grp0, const bool near60, const int dshift = 0,
                                           const uint64_t dmask = ~0ULL) {
-    if (kb_fold_prime(mods[m]))  // uniform: one modulus per workgroup
+    if (near60)  // uniform: one modulus per workgroup
         pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, DIG, true>(tile, in, out, tw, ninv_tab, w1_tab, mods, m,
                                                                         grp0, dshift, dmask);
     else
@@ -400,10 +400,24 @@ __device__ __forceinline__ void pass_body(uint64_t *tile, const uint64_t *__rest
 
 // XCD-aware order: workgroup b runs on XCD b % 8, so when the grid is a
 // multiple of 8 each XCD gets a contiguous range of tiles (the column tiles
-// that share DRAM rows, and one modulus' twiddles, stay in one L2)
+// that share DRAM rows, and one modulus' twiddles, stay in one L2).  xcd: an eighth of the
+// grid (an argument: gridDim is one more read of host memory), 0 for the launch order
 __device__ __forceinline__ int xcd_block(int xcd) {
-    if (xcd && (gridDim.x & 7) == 0) return (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+    if (xcd) return (int)(blockIdx.x & 7) * xcd + (int)(blockIdx.x >> 3);
     return (int)blockIdx.x;
+}
+int xcd_eighth(long blocks, int ordered) { return ordered && blocks % 8 == 0 ? (int)(blocks / 8) : 0; }
+
+// Bit m for a modulus near 2^60 (an argument: no load of the modulus stands before the
+// tile's and the twiddles' loads)
+struct kind_bits {
+    uint64_t w[3];
+    __device__ __forceinline__ bool at(int m) const { return (m < 64 ? w[0] : m < 128 ? w[1] : w[2]) >> (m & 63) & 1; }
+};
+kind_bits kinds_of(const kbfv_context *c) {
+    kind_bits k{};
+    for (int m = 0; m < c->nmod; ++m) k.w[m >> 6] |= (uint64_t)kb_fold_prime(c->mod[m]) << (m & 63);
+    return k;
 }
 
 // the moduli of a launch: none near 2^60, all, or some of each.  The kernel for some of
@@ -412,14 +426,16 @@ __device__ __forceinline__ int xcd_block(int xcd) {
 // launches only.
 enum { SHOUP, FOLD, BOTH };
 
-// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL
-template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, int KIND>
+// strided batch: limb l of polynomial y of batch entry bi at src + bi*sB + y*sY + l*sL;
+// PAIR: entries from `half` on come from src2 (its arguments cost the other launches 0.4 us,
+// a wait for host memory, where 48 limbs take 8)
+template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD, bool NOSCALE, int KIND, bool PAIR>
 __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     k_ntt_pass(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
                const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
                const kbfv_tw *__restrict__ w1_tab, const uint64_t *__restrict__ mods, int mod0, int limbs,
                int polys, int batch, long sB, long sY, long sL, long dB, long dY, long dL, int xcd,
-               const uint64_t *__restrict__ src2, int half) {
+               const uint64_t *__restrict__ src2, int half, kind_bits kinds) {
     using G = Geo<LOG_S, COLUMN, LOG_T>;
     constexpr int groups = (1 << (LOG_N - LOG_S)) / G::C;  // workgroups per limb
     __shared__ uint64_t tile[G::WORDS];
@@ -430,10 +446,11 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     bid /= polys;
     const int bi = bid % batch;
     const int l = bid / batch;
-    const uint64_t *in = (bi < half ? src + bi * sB : src2 + (bi - half) * sB) + y * sY + l * sL;
+    const uint64_t *in = (PAIR && bi >= half ? src2 + (bi - half) * sB : src + bi * sB) + y * sY + l * sL;
     uint64_t *out = dst + bi * dB + y * dY + l * dL;
     if constexpr (KIND == BOTH)
-        pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, in, out, tw, ninv_tab, w1_tab, mods, mod0 + l, grp0);
+        pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE>(tile, in, out, tw, ninv_tab, w1_tab, mods, mod0 + l, grp0,
+                                                             kinds.at(mod0 + l));
     else
         pass_tile<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, false, KIND == FOLD>(tile, in, out, tw, ninv_tab, w1_tab,
                                                                                   mods, mod0 + l, grp0);
@@ -545,7 +562,7 @@ template <int LOG_N, int LOG_S, int LOG_T, bool COLUMN, bool FWD>
 __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     k_ntt_pass_desc(const int64_t *__restrict__ desc, const int32_t *__restrict__ limb_start, int count,
                     int in_dst, const kbfv_tw *__restrict__ tw, const kbfv_tw *__restrict__ ninv_tab,
-                    const uint64_t *__restrict__ mods, int xcd) {
+                    const uint64_t *__restrict__ mods, int xcd, kind_bits kinds) {
     using G = Geo<LOG_S, COLUMN, LOG_T>;
     constexpr int groups = (1 << (LOG_N - LOG_S)) / G::C;
     __shared__ uint64_t tile[G::WORDS];
@@ -566,8 +583,9 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     if (l >= d[5]) return;  // a total past the uploaded one: uniform per workgroup, before any barrier
     uint64_t *dst = (uint64_t *)d[1];
     const uint64_t *in = in_dst ? dst + l * d[3] : (const uint64_t *)d[0] + l * d[2];
-    pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, false>(tile, in, dst + l * d[3], tw, ninv_tab, ninv_tab, mods,
-                                                       (int)d[4] + (int)l, grp0);
+    const int m = (int)d[4] + (int)l;
+    pass_body<LOG_N, LOG_S, LOG_T, COLUMN, FWD, false>(tile, in, dst + l * d[3], tw, ninv_tab, ninv_tab, mods, m, grp0,
+                                                       kinds.at(m));
 }
 
 struct pass_args {
@@ -600,12 +618,17 @@ int launch_pass(const pass_args &a) {
         const long groups = (1L << (LOG_N - LOG_S)) / G::C;
         const long blocks = groups * a.limbs * a.polys * a.batch;
         KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
+        const auto launch = [&](auto kind, auto pair) {
+            hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, decltype(kind)::value,
+                                           decltype(pair)::value>),
+                               dim3((unsigned)blocks), dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv,
+                               a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB,
+                               a.dY, a.dL, xcd_eighth(blocks, a.xcd), a.src2, a.half, MIXED ? kinds_of(a.c) : kind_bits{});
+        };
         const auto go = [&](auto kind) {
-            constexpr int KIND = decltype(kind)::value;
-            hipLaunchKernelGGL((k_ntt_pass<LOG_N, LOG_S, LOG_T, COLUMN, FWD, NOSCALE, KIND>), dim3((unsigned)blocks),
-                               dim3(G::T), 0, a.st, a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod,
-                               a.mod0, a.limbs, a.polys, a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd, a.src2,
-                               a.half);
+            if constexpr (!COLUMN && !FWD)  // the first pass of a transform from two sources
+                if (a.src2) return launch(kind, std::true_type{});
+            launch(kind, std::false_type{});
         };
         if constexpr (MIXED)
             go(std::integral_constant<int, BOTH>{});
@@ -786,7 +809,8 @@ __global__ void __launch_bounds__((1 << LOG_T) >> LOG_R)
     const uint64_t *in = coef + bt * 2 * L + (long)(row / nd) * n;  // (h*qn + i)*N = h*L + i*N
     uint64_t *out = dig + (bt * rc + y) * L + (long)l * n;
     pass_body<LOG_N, LOG_S, LOG_T, true, true, false, true>(tile, in, out, tw, nullptr, nullptr, mods, oQ + l, grp0,
-                                                            bits * (row % nd), (1ULL << bits) - 1);
+                                                            kb_fold_prime(mods[oQ + l]), bits * (row % nd),
+                                                            (1ULL << bits) - 1);
 }
 
 // ---------------------------------------------------------------- plans
@@ -848,7 +872,7 @@ int launch_limb(const pass_args &a) {
     KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
     hipLaunchKernelGGL((k_ntt_limb<LOG_N, FWD, NOSCALE>), dim3((unsigned)blocks), dim3((1 << LOG_N) >> LOG_R), 0, a.st,
                        a.src, a.dst, a.c->t.tw, a.c->t.ninv, a.c->t.inv_w1, a.c->t.mod, a.mod0, a.limbs, a.polys,
-                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, a.xcd, a.src2, a.half);
+                       a.batch, a.sB, a.sY, a.sL, a.dB, a.dY, a.dL, xcd_eighth(blocks, a.xcd), a.src2, a.half);
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }
@@ -1018,7 +1042,7 @@ int launch_digit_col(const kbfv_context *c, int log_t, const uint64_t *coef, uin
             const long blocks = (long)c->qn * ((1L << (LOG_N - LOG_S)) / G::C) * rc * batch;
             KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
             hipLaunchKernelGGL((k_ntt_digit_col<LOG_N, LOG_S, LT>), dim3((unsigned)blocks), dim3(G::T), 0, st, coef,
-                               dig, c->t.tw, c->t.mod, c->oQ, c->qn, nd, bits, r0, rc, 1);
+                               dig, c->t.tw, c->t.mod, c->oQ, c->qn, nd, bits, r0, rc, xcd_eighth(blocks, 1));
             KB_LAUNCH_CHECK();
             return KBFV_OK;
         }
@@ -1236,7 +1260,7 @@ int launch_desc(const kbfv_context *c, const int64_t *desc, const int32_t *start
     const long blocks = (long)total * ((1L << (LOG_N - LOG_S)) / G::C);
     KB_REQUIRE(blocks < (1L << 31), "NTT grid too large");
     hipLaunchKernelGGL((k_ntt_pass_desc<LOG_N, LOG_S, 12, COLUMN, FWD>), dim3((unsigned)blocks), dim3(G::T), 0, st,
-                       desc, start, count, in_dst, c->t.tw, c->t.ninv, c->t.mod, 1);
+                       desc, start, count, in_dst, c->t.tw, c->t.ninv, c->t.mod, xcd_eighth(blocks, 1), kinds_of(c));
     KB_LAUNCH_CHECK();
     return KBFV_OK;
 }

@@ -11,6 +11,8 @@
 // MI355X design: with one special prime (K = 1) the digit decomposition of a
 // limb is the limb itself, so "modUp Qj -> T then NTT over T" is one NTT that
 // reads the Q limb directly (kb_digits_to_t_ntt).
+#include <algorithm>
+
 #include "kbfv_internal.h"
 #include "kbfv_ops.h"
 
@@ -170,29 +172,33 @@ __global__ void k_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint
 // in registers.  NOSC: the input is N times the INTT (lazy, below 4t); the
 // first step [(x + T/2) (T/t)^-1]_t is a Shoup product exact for any 64-bit
 // operand, so it takes ([N T/2]_t, [(T/t)^-1 n^-1]_t) instead and gives the
-// same canonical value.  grid (n / KS_BS, batch * 2)
+// same canonical value.  grid (n / KS_BS, batch * 2, slices of `per` ri blocks): a slice
+// past the first takes the P residues from block 0 for itself.
 template <int TN, int G, int PN, bool NOSC>
 __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
                                 const uint64_t *__restrict__ add, long add_stride, int add_h, int qn, int B,
-                                int oQ, int oT, int n) {
+                                int per, int oQ, int oT, int n) {
+    static_assert(PN <= G, "block 0 holds the P limbs");
     const int k = blockIdx.x * KS_BS + threadIdx.x;
     const long rest = blockIdx.y;
     const int h = (int)(rest & 1);
     const long bt = rest >> 1;
     const int pq = PN + qn;
+    const int b0 = (int)blockIdx.z * per, b1 = min(b0 + per, B);
     uint64_t xp[PN];  // the P residues of this coefficient
-    // the T values of ri block b + 1 are loaded while block b is converted
+    // the T values of the next ri block are loaded while block b is converted
     const uint64_t *ip0 = in + rest * B * (long)TN * n + k;
     uint64_t nxt[TN];
 #pragma unroll
     for (int kk = 0; kk < TN; ++kk) nxt[kk] = ip0[(long)kk * n];
-    for (int b = 0; b < B; ++b) {
+    for (int b = 0, next; b < b1; b = next) {
+        next = max(b + 1, b0);
         uint64_t cur[TN];
 #pragma unroll
         for (int kk = 0; kk < TN; ++kk) cur[kk] = nxt[kk];
-        if (b + 1 < B) {
+        if (next < b1) {
 #pragma unroll
-            for (int kk = 0; kk < TN; ++kk) nxt[kk] = ip0[((long)(b + 1) * TN + kk) * n];
+            for (int kk = 0; kk < TN; ++kk) nxt[kk] = ip0[((long)next * TN + kk) * n];
         }
         uint64_t rb[TN];
         float vv = 0;
@@ -209,7 +215,7 @@ __global__ void k_modup_moddown(kb_dev_tables t, const uint64_t *__restrict__ in
 #pragma unroll
         for (int j = 0; j < G; ++j) {
             const int idx = b * G + j;
-            if (idx >= pq) break;
+            if (idx >= pq || (b < b0 && idx >= PN)) break;
             const uint64_t r = t.mod[idx];
             kbfv_u128 acc{0, 0};
 #pragma unroll
@@ -263,12 +269,19 @@ static int modup_moddown(const kbfv_context *c, const uint64_t *in, uint64_t *ou
                          long add_stride, int add_h, int batch, uint64_t *pq_tmp, bool nosc, hipStream_t st) {
     KB_REQUIRE(c && in && out && batch > 0, "bad modUp/modDown arguments");
     KB_REQUIRE(2L * batch <= 65535, "batch too large for one modUp/modDown launch");
+    // Few coefficients leave the chip idle while a thread walks its blocks: they are split
+    // over up to eight. Whole / split, the call with its transforms, us: 28 primes, N=4096, 1
+    // ciphertext 54/28 (8), N=2^16, 1 147/135 (3), 2 253/244 (3), 4 465/452 (3); two special primes
+    // and 12 others, 2^15, 1 66/52 (4), 2 87/80 (3), 4 124/123 (3), 8 239/243 (3)
+    const long waves = (long)c->n * 2 * batch / 64;
+    const int slices = (int)std::max(1L, std::min({8L, (c->ri_blocks + 1L) / 2, 6144 / waves}));
+    const int per = (c->ri_blocks + slices - 1) / slices;
     // PN special residues first: the P limbs must all lie before any Q limb
 #define KB_MUMD(TN_, G_, PN_, NOSC_)                                                                       \
     if (c->tn == TN_ && c->gamma == G_ && c->pn == PN_ && nosc == NOSC_) {                                 \
-        hipLaunchKernelGGL((k_modup_moddown<TN_, G_, PN_, NOSC_>), dim3(c->n / KS_BS, 2 * batch), dim3(KS_BS), \
-                           0, st, c->t, in, out, add, add_stride, add_h, c->qn, c->ri_blocks, c->oQ, c->oT,  \
-                           c->n);                                                                            \
+        hipLaunchKernelGGL((k_modup_moddown<TN_, G_, PN_, NOSC_>),                                         \
+                           dim3(c->n / KS_BS, 2 * batch, (c->ri_blocks + per - 1) / per), dim3(KS_BS), 0, st, \
+                           c->t, in, out, add, add_stride, add_h, c->qn, c->ri_blocks, per, c->oQ, c->oT, c->n); \
         KB_LAUNCH_CHECK();                                                                                 \
         return KBFV_OK;                                                                                    \
     }

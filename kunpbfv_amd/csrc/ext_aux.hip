@@ -23,11 +23,11 @@
 // accumulates with one v_mad_u64_u32 per product and reduces once.
 //
 // 128 products at N = 2^16, 28 primes, base 2^20 (168 rows, four auxiliary primes):
-// 84.8 ms against 422 ms through 4704 60-bit transforms per ciphertext; of
-// that the row products 31, the digits' transforms 20, the rows' basis
-// change 15, the way back and the ciphertext's own transforms 18.  The row products
-// wait on LDS and on one another's stages: two waves per SIMD issue a multiply-add
-// in about half the slots.
+// 81 ms against 422 ms through 4704 60-bit transforms per ciphertext; of that the row
+// products 31.6, the transforms of digits and rows in the basis 29.7, the way back 9.5, the
+// 60-bit transforms of ciphertexts, rows and results 10.2.  The row products hold seven waves
+// per CU and issue 0.42 VALU instructions per clock and CU, half of what multiply-adds
+// reach; a fifth of the waves' time is spent waiting, a third of that on LDS.
 #include <algorithm>
 #include <cmath>
 

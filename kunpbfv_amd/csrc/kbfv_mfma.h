@@ -11,11 +11,9 @@
 // digit v = w - u of m_k.  With r = bytereverse(digits(m_k)) that operand is just
 // r shifted by 8|w - 7| bits (left for w > 7, right for w < 7), zero bytes where
 // w - u leaves [0, 7].  |P_w| <= 8 K 2^14, so int32 accumulation is exact for
-// K <= 2^14; the sum is rebuilt as
-//     sum_w P_w 2^(8w) = (S2 2^48 + S1) 2^48 + S0,
-//     S2 = P_14..P_12, S1 = P_11..P_6, S0 = P_5..P_0 (Horner in 2^8, int64),
-// which is exact in 128-bit wrap-around arithmetic because the true value is a
-// non-negative integer below 2^127.
+// K <= 2^14; biased like the sums below, pairs of them combine into 32-bit words, which
+// rebuild the sum exactly in 128 bits because the true value is a non-negative integer
+// below 2^127.
 //
 // Constant matrices use an expanded form instead: since x = sum_u d_u 2^(8u),
 //     sum_k x_k m_k = sum_(k,u) d_ku (2^(8u) m_k mod p)   (mod p),
@@ -25,8 +23,8 @@
 // accumulators A_v in [0, 2^23] (KB_MX_ACC_BIAS) the sum is
 //     V = sum_v A_v 2^(8v) + off,   off = (-bias sum_v 2^(8v)) mod p,
 // a non-negative integer below 2^80 congruent to the dot product; the four
-// 32-bit words A_(2k+1) 2^8 + A_2k give V exactly mod 2^64 and, in double
-// precision, a quotient estimate that is one of floor(V/p) - 1, floor(V/p)
+// 32-bit words A_(2k+1) 2^8 + A_2k give V exactly.  Its top 32 bits times
+// floor(2^(80+S)/p) (KB_MX_QSHIFT), a 32-bit high product, are floor(V/p) or one less
 // for p >= 2^58, so one multiply-subtract and one conditional subtraction
 // finish the reduction.
 //
@@ -75,13 +73,3 @@ __device__ __forceinline__ uint64_t kb_weight_op(uint64_t r, int w) {
 __device__ __forceinline__ kb_v4i kb_mfma_i8(kb_v4i a, kb_v4i b, kb_v4i c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
-
-// (hi:lo) = (hi:lo) * 2^48 + s  (s signed)
-__device__ __forceinline__ void kb_horner48(uint64_t &lo, uint64_t &hi, int64_t s) {
-    hi = (hi << 48) | (lo >> 16);
-    lo <<= 48;
-    const uint64_t nl = lo + (uint64_t)s;
-    hi += (uint64_t)(nl < lo) + (s < 0 ? ~0ULL : 0ULL);
-    lo = nl;
-}
-

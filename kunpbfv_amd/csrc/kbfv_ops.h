@@ -35,7 +35,8 @@ int kb_modup_qj_to_t(const kbfv_context *c, const uint64_t *x, long xs, uint64_t
 int kb_modup_pq_to_t(const kbfv_context *c, const uint64_t *x, uint64_t *out, int batch, hipStream_t st);
 int kb_inner_product(const kbfv_context *c, const uint64_t *cin, const uint64_t *key, uint64_t *out,
                      int batch, hipStream_t st);
-// ks_ip.hip: the inner product with the key streamed, for small batches
+// ks_ip.hip: the inner product on the VALU, the key streamed past one to four ciphertexts
+// or held in registers for more
 int kb_inner_product_stream(const kbfv_context *c, const uint64_t *cin, const uint64_t *key, uint64_t *out, int batch,
                             hipStream_t st);
 // ks_mfma.hip: the inner product on the int8 matrix cores (returns 1 when the

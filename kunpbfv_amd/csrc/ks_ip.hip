@@ -1,9 +1,10 @@
-// Key-switch inner product for small batches: the key streams past.
+// Key-switch inner product on the VALU: the key streams past one to four ciphertexts
+// (k_ip_stream) or stays in registers while more walk by (k_ip_hold, up to 32 digits).
 //
 // Replaces external_product_T_kernel and its _swk_reuse variant
 // (include/ExternalProduct.cuh:11-177): for T limb k and coefficient n,
 //     out[ct][h][b] = sum_{d < D} cin[ct][d] key[h][d][b]   mod t_k.
-// A thread takes V coefficients of one key block b, both key halves h, and C
+// In the stream a thread takes V coefficients of one key block b, both key halves h, and C
 // ciphertexts at a time; a workgroup's waves take neighbouring blocks of the same
 // coefficients, so the digits they share come through one L1.
 //

@@ -6,6 +6,10 @@
 // psi[m + group]), Gentleman-Sande inverse with the bit-reversed psi^-1 table
 // whose entry 1 carries n^-1, outputs canonical in [0, q).
 //
+// Three families of kernels, by primes and size: many limbs of primes near 2^60 take
+// the one-pass kernel (ntt_reg.hip), up to 2^19 words k_ntt_small, the rest, and explicit
+// plans, the tile passes described here.
+//
 // Design (MI355X): N = N1 * N2 four-step split into two passes, each a kernel
 // that stages a tile of 2^11-2^13 elements (16-64 KiB, the plan's choice) in
 // LDS and runs radix-16 rounds in registers:

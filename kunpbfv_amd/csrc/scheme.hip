@@ -1021,7 +1021,7 @@ extern "C" int kbfv_external_product(const kbfv_context *c, const uint64_t *rgsw
     // The auxiliary basis costs a basis change of the whole RGSW ciphertext, which enough
     // ciphertexts have to share, fewer the more words one polynomial has to keep the chip
     // busy with.  General / auxiliary path, base 2^20, us: N=2^16, 28 primes, 8
-    // ciphertexts 27500/31600, 12 40600/31500; 12 of 50 bits, 11 ciphertexts 6900/6800, 12
+    // ciphertexts 27500/31600, 12 40600/31500; 12 of 50 bits, 10 ciphertexts 6343/6574, 12
     // 7524/7001; 9 primes, 12 3901/4370, 13 4285/4323, 14 4640/4332; 2^15, 13 primes, 12
     // 4224/4351, 13 4612/4228; 9 primes, 14 2386/2528, 15 2568/2371; 2^14, 12 primes, 16
     // 2247/2379, 17 2470/2239; 2^13, 8 of 45 bits, 17 777/831, 20 886/705; 2^12, 4 primes, 16

@@ -31,7 +31,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # 4 GiB device copy in the same run.  A plan without a recorded profile
 # reports traffic null rather than a figure measured for another plan.
 NTT_TRAFFIC = {
-    (16, 28, 128, 0x3cd8): (2 * 23_000_583_594, "profiles/ntt_qr_inverse_n65536_b128_counters.md"),
+    (16, 28, 128, 0x3cc8): (44_703_361_518, "profiles/ntt_qr_inverse_n65536_b128_counters.md"),
 }
 
 

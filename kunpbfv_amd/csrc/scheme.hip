@@ -1028,10 +1028,13 @@ extern "C" int kbfv_external_product(const kbfv_context *c, const uint64_t *rgsw
     // 251/266, 20 305/234.  Short chains gain less, as a digit has as many transforms there
     // as here: 4 primes at 2^16, 25 1653/1644; 3 there, 64 2625/2812; 2 at 2^15, 100
     // 1395/1514, at 2^14, 50 432/407; 1 at 2^14, 200 691/815, at 2^13, 128 399/386, 100 320/340.
-    const int least = L >= 3L << 18 ? 12 : L >= 3L << 17 ? 13 : L >= 7L << 15 ? 15 : L >= 5L << 15 || qn > 16 ? 17 : 18;
-    const bool enough = batch >= least && batch * (long)qn >= (qn == 1 && c->log_n > 12 ? 112 : 100) &&
-                        qn >= c->log_n - 12;
-    const int np = enough ? kb_ext_aux_primes(c, rows, base_bits) : 0;
+    // Three auxiliary primes (short primes, small bases) reach it a little earlier: 13 of 45 bits
+    // at 2^12, base 2^10, 17 1838/1427; 1 at 2^13, base 2^4, 100 1437/982.
+    const int most = batch >= 12 && batch * (long)qn >= 100 ? kb_ext_aux_primes(c, rows, base_bits) : 0;
+    int least = most < 4 || qn > 16 || L >= 5L << 15 ? 17 : 18;
+    if (L >= 7L << 15) least = L >= 3L << 18 ? 12 : L >= 3L << 17 ? 13 : 15;
+    const bool enough = batch >= least && qn >= c->log_n - 12 && (qn > 1 || c->log_n == 12 || most < 4 || batch >= 112);
+    const int np = enough ? most : 0;
     if (np && kb_ext_aux_rows(c, batch, np) >= 1)
         return kb_external_product_aux(c, rgsw, coef, out, dig, batch, rows, nd, base_bits, np, s);
     KB_TRY(fill_zero(out, 2 * L * batch, s));
